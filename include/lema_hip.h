@@ -102,6 +102,18 @@ int lema_gather(const void* v, int32_t dtype, int64_t B, int64_t H, int64_t T, i
                 void* y, int64_t y_sb, int64_t y_sh, int64_t y_st, int32_t miss,
                 void* stream);
 
+/* The gradient of the gather: gv[b, h, j, :] = sum of gy[b, h, i, :] over the queries i with
+ * src[b, h, i] = j, summed in fp32 and rounded once (16-bit types: once per 1536 or more listed
+ * queries of 1024 rows). A missed query's row times zero counts towards row 0, so an infinity
+ * or NaN there makes that column of gv[b, h, 0] NaN. Replaces the backward of
+ * code/lema/attention.py:157-158.
+ *   gy   [B, H, T, dv] of `dtype`, element strides (any, zero included), last dim contiguous
+ *   src  contiguous int32 [B*H, T], every entry in [-1, T) and below its own position
+ *   gv   contiguous [B, H, T, dv] of `dtype`, written whole                               */
+int lema_gather_grad(const void* gy, int32_t dtype, int64_t B, int64_t H, int64_t T, int64_t dv,
+                     int64_t gy_sb, int64_t gy_sh, int64_t gy_st, const int32_t* src, void* gv,
+                     void* stream);
+
 /* One exchange against the shared open-addressing store in device memory.
  * Replaces store_exchange, code/lema/csrc/store.cpp:122-162 (bound as lema_store.exchange,
  * store.cpp:164-167, called from HashStore.exchange, code/lema/cache.py:184-201).

@@ -192,6 +192,19 @@ def gather_values(v: torch.Tensor, src: torch.Tensor, miss: str = "dense") -> to
     return y
 
 
+def _plain_grad(gy: torch.Tensor) -> bool:
+    """Whether a backward may hand gy to the kernel: an ordinary device tensor whose own
+    gradient nobody asks for. A graph of the backward (create_graph), forward mode, batched
+    gradients and traced or otherwise wrapped tensors keep the tensor operations, which
+    compose with them or refuse them by themselves."""
+    ft = torch._C._functorch
+    return (type(gy) is torch.Tensor and gy.is_cuda and gy.dtype in _lib.DTYPE_CODE
+            and not torch.is_grad_enabled() and torch._C._len_torch_dispatch_stack() == 0
+            and not ft.is_functorch_wrapped_tensor(gy) and not ft.is_legacy_batchedtensor(gy)
+            and torch.autograd.forward_ad._current_level < 0
+            and not gy.is_neg() and not gy._is_zerotensor())
+
+
 class _LemaGather(torch.autograd.Function):
     """The value path stays differentiable (code/lema/attention.py:146-148): the gradient
     of y = v[src] * (src >= 0) sends each dy row to its source row."""
@@ -207,6 +220,14 @@ class _LemaGather(torch.autograd.Function):
     def backward(ctx, gy):
         (src,) = ctx.saved_tensors
         B, H, T, dv = ctx.v_shape
+        if _plain_grad(gy):
+            gy = gy if gy.stride(-1) == 1 or dv == 1 else gy.contiguous()
+            gv = torch.empty((B, H, T, dv), dtype=gy.dtype, device=gy.device)
+            _lib.check(_lib.lib().lema_gather_grad(
+                gy.data_ptr(), _lib.DTYPE_CODE[gy.dtype], B, H, T, dv, gy.stride(0),
+                gy.stride(1), gy.stride(2), src.contiguous().data_ptr(), gv.data_ptr(),
+                _lib.stream_of(gy)))
+            return None, None, gv
         hit = (src >= 0).unsqueeze(-1)
         idx = src.clamp_min(0).to(torch.int64).view(B * H, T, 1).expand(B * H, T, dv)
         gv = torch.zeros((B * H, T, dv), dtype=gy.dtype, device=gy.device)
