@@ -75,7 +75,7 @@ int lema_hard(const void* qc, const void* kc, int32_t code_bytes, const void* v,
               int32_t miss, void* src, int32_t src_bytes, void* stream);
 
 /* Workspace bytes lema_latest_prev_match_ws and lema_hard_ws use for N rows of T positions:
- * 8 KB per 1024 positions, 0 for rows of fewer than 64,513 positions (64 chunks of 1024;
+ * about 24 KB per 1024 positions, 0 for rows of fewer than 64,513 positions (64 chunks of 1024;
  * shorter rows keep the backward scan, which is faster there, and need none). No reference counterpart: the reference's sort needs no scratch the
  * caller provides. */
 int64_t lema_resolve_workspace_bytes(int64_t N, int64_t T);

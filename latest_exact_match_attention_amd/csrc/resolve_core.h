@@ -88,6 +88,11 @@ constexpr int kScanGroup = 4;  // key batches whose loads the queued scan issues
 // find their latest key a few chunks back, where the summaries win (16 x 262144: 441 against
 // 879 us).
 constexpr int kQueueSummMinCodes = 896;
+// The bits of mask_hash leave a code that has no earlier key only the 1.6% of chunks that hold
+// its hash, so from chunk kQueueSummChunks on the summaries win for such codes too (24 rows x
+// T = 100003: 141 against 487 us; below it the scan: 32 x 65536, 105 us against 133 with the
+// line at chunk 48).
+constexpr int kQueueSummChunks = 64;
 // The scan tests every earlier key with it, so it avoids the quarter-rate 32-bit multiply:
 // the high half is folded into the low 24 bits, which a full-rate 24-bit multiply mixes.
 // (__umul24 is declared to return int: the product is shifted as unsigned.)
@@ -244,6 +249,12 @@ struct ResolveArgs {
   // scanning every earlier key.
   uint32_t* summ_tab;
   int32_t* summ_sent;
+  uint32_t* summ_bits;  // per (row, chunk): bit mask_hash(c) of every key code c of the chunk
+  uint64_t* summ_mask;  // the same turned round, per (row, hash): bit k = chunk k of the row
+                        // holds such a key, mask_words 64-bit words
+  uint16_t* summ_lone;  // per (row, chunk): of kLoneSample queries, those with no key there
+  uint8_t* mask_built;  // per row: 1 = summ_mask holds its bits
+  int32_t mask_words;
   int32_t group;  // workgroup order: 8 consecutive rows per XCD, one chunk of all 8 in a row
   GatherArgs g;
 };
@@ -294,11 +305,34 @@ __device__ __forceinline__ int32_t summary_probe(const uint32_t* tab, const Code
   }
 }
 
+// Which chunks of a row may hold a code: one bit per (hash of the code, chunk), read as one run
+// of bits per code. A chunk sets at most 1024 of the 65,536 bits, so a code is looked up in
+// the few chunks that do hold it and in 1.6% of the others, instead of in every earlier chunk
+// until one holds it: 24 rows x T = 262144 of 64-bit codes over 30,000 values with a quarter
+// of the queries never matched took 1811 us that way (rate of the tables' 16-byte reads).
+constexpr int kMaskLog2 = 16;
+constexpr int kMaskWords = (1 << kMaskLog2) / 32;  // summ_bits words per chunk
+// The bits pay where many queries carry codes that the nearest chunks don't hold. summary_kernel
+// looks kLoneSample of a chunk's queries up among the chunk's own keys; a row gets its bits when
+// more than kLoneRow of them (22%) have none there, on average. Codes that repeat more than
+// that are found a chunk or two back without them (24 x T = 262144 of 32-bit codes, over 600
+// values, 18%: 164 us without, 193 with; over Zipf 4096, 27%: 587 and 261). A chunk of at most kLoneChunk (20%)
+// leaves its bits out and counts as holding every code. In rows of up to kMaskQueueChunks
+// chunks the queries of codes that hardly ever repeat (more than kLoneQueue, 90%) take the
+// queued scan instead (32 rows x T = 65536 of uniform codes: 105 us without bits, 121 with).
+constexpr int kLoneSample = 256, kLoneRow = 56, kLoneChunk = 52, kLoneQueue = 230;
+constexpr int kMaskQueueChunks = 72;
+__device__ __forceinline__ uint32_t mask_hash(uint32_t h) {
+  return ((h ^ (h >> 15)) * 0x2C1B3C6Du) >> (32 - kMaskLog2);
+}
+
 // Latest key position before chunk `chunk` of row `row` for code x (sent: x is the all-ones
-// code), or -1: the summaries of the earlier chunks are probed latest first, 8 at a time
-// with their first buckets loaded together.
+// code), or -1: the summaries of the earlier chunks are probed latest first, 8 at a time with
+// their first buckets loaded together; with the row's bits (`masked`) only those of chunks that
+// may hold x, 4 at a time.
 template <typename CodeT>
-__device__ __forceinline__ int32_t before_chunk(const ResolveArgs& a, int64_t row, int chunk, CodeT x, bool sent) {
+__device__ __forceinline__ int32_t before_chunk(const ResolveArgs& a, int64_t row, int chunk, CodeT x, bool sent,
+                                                bool masked) {
   constexpr int kAhead = 8;
   const int64_t rc = row * a.nchunks;
   if (sent) {
@@ -315,21 +349,53 @@ __device__ __forceinline__ int32_t before_chunk(const ResolveArgs& a, int64_t ro
   const CodeT* krow = static_cast<const CodeT*>(a.kc) + row * a.T;
   const uint32_t fp = fingerprint(fold(x));
   const int b0 = bucket_of<kSumBuckets>(fold(x));
-  for (int cb = chunk - 1; cb >= 0; cb -= kAhead) {
-    u32x4 e[kAhead];
+  if (!masked) {
+    for (int cb = chunk - 1; cb >= 0; cb -= kAhead) {
+      u32x4 e[kAhead];
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i)
-      e[i] = cb - i >= 0 ? *reinterpret_cast<const u32x4*>(a.summ_tab + (rc + cb - i) * kSumSlots + 4 * b0)
-                         : u32x4{kSumEmpty, kSumEmpty, kSumEmpty, kSumEmpty};
+      for (int i = 0; i < kAhead; ++i)
+        e[i] = cb - i >= 0 ? *reinterpret_cast<const u32x4*>(a.summ_tab + (rc + cb - i) * kSumSlots + 4 * b0)
+                           : u32x4{kSumEmpty, kSumEmpty, kSumEmpty, kSumEmpty};
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      if (cb - i < 0) break;
-      const int32_t j = summary_probe(a.summ_tab + (rc + cb - i) * kSumSlots, krow, cb - i, x,
-                                      fp, b0, e[i]);
+      for (int i = 0; i < kAhead; ++i) {
+        if (cb - i < 0) break;
+        const int32_t j = summary_probe(a.summ_tab + (rc + cb - i) * kSumSlots, krow, cb - i, x,
+                                        fp, b0, e[i]);
+        if (j >= 0) return j;
+      }
+    }
+    return -1;
+  }
+  const uint64_t* mask = a.summ_mask + ((row << kMaskLog2) + mask_hash(fold(x))) * a.mask_words;
+  int wi = (chunk - 1) >> 6;
+  uint64_t cur = mask[wi] & (~0ull >> (63 - ((chunk - 1) & 63)));
+  uint64_t nxt = wi > 0 ? mask[wi - 1] : 0;  // read ahead of its use
+  constexpr int kTry = 4;
+  for (;;) {
+    int cc[kTry];
+    u32x4 e[kTry];
+#pragma unroll
+    for (int i = 0; i < kTry; ++i) {
+      while (cur == 0 && wi > 0) {
+        --wi;
+        cur = nxt;
+        nxt = wi > 0 ? mask[wi - 1] : 0;
+      }
+      cc[i] = -1;
+      if (cur != 0) {
+        const int b = 63 - __clzll(cur);
+        cur ^= 1ull << b;
+        cc[i] = (wi << 6) + b;
+        e[i] = *reinterpret_cast<const u32x4*>(a.summ_tab + (rc + cc[i]) * kSumSlots + 4 * b0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kTry; ++i) {
+      if (cc[i] < 0) return -1;
+      const int32_t j = summary_probe(a.summ_tab + (rc + cc[i]) * kSumSlots, krow, cc[i], x, fp, b0, e[i]);
       if (j >= 0) return j;
     }
   }
-  return -1;
 }
 
 // ------------------------------------------------------------------ miss fill (dense path)
@@ -949,9 +1015,11 @@ __device__ __forceinline__ void resolve_chunk(ResolveLds<CodeT>& s, const Resolv
         if (s.pos[x] == -2) need[atomicAdd(&s.nneed, 1)] = x;
       bar();
       const int nneed = s.nneed;
+      const bool masked = a.mask_built[row] != 0;
       for (int i = t; i < nneed; i += kThreads) {
         const int x = need[i];
-        s.pos[x] = before_chunk<CodeT>(a, row, chunk, x == kSlots ? SENT : s.code[x], x == kSlots);
+        s.pos[x] = before_chunk<CodeT>(a, row, chunk, x == kSlots ? SENT : s.code[x], x == kSlots,
+                                        masked);
       }
       bar();
 #pragma unroll
@@ -973,7 +1041,7 @@ __device__ __forceinline__ void resolve_chunk(ResolveLds<CodeT>& s, const Resolv
   if (!filt) {
     rest(std::false_type{}, std::false_type{});
   } else if constexpr (kSumm) {
-    if (s.nq > kQueueSummMinCodes)
+    if (s.nq > kQueueSummMinCodes && (chunk < kQueueSummChunks || a.mask_built[row] == 0))
       rest(std::true_type{}, std::true_type{});
     else
       rest(std::true_type{}, std::false_type{});

@@ -676,3 +676,36 @@ def test_queued_scan_high_cardinality_rows(dev, code_dtype):
     _, src = lema_from_codes(q.view(1, N, T), k.view(1, N, T), v, return_src=True)
     assert np.array_equal(src.cpu().numpy().reshape(N, T).astype(np.int64), want)
     assert (want[0] >= 0).sum() > 1500 and (want[1] >= 0).sum() > 1500
+
+
+@pytest.mark.parametrize("T", [66 * 1024 + 5, 73 * 1024, 130 * 1024 + 700])
+@pytest.mark.parametrize("kind", ["few", "lone", "uniform", "late", "mixed"])
+def test_chunk_bits(dev, T, kind):
+    """Long rows with and without the per-code chunk bits: keys of few codes (no bits), a
+    quarter of the queries with no key (bits; the row's 64-chunk words and the line between the
+    bits and the queued scan crossed), uniform codes, codes whose only key lies far back, and
+    rows where half of the chunks leave their bits out. Against the scan without a workspace."""
+    from latest_exact_match_attention_amd import _lib, attention
+    g = torch.Generator().manual_seed(T)
+    N = 3
+    qc, kc = (torch.randint(0, 400, (N, T), generator=g) for _ in range(2))
+    lone = torch.rand((N, T), generator=g) < 0.25
+    at = torch.arange(T).expand(N, T)
+    if kind in ("lone", "late"):
+        qc = torch.where(lone, 1000 + at, qc)
+    if kind == "late":       # half of those codes do have a key, in the row's first chunks
+        kc[:, :3000] = 1000 + T - 1 - torch.randperm(T, generator=g)[:3000]
+    if kind == "uniform":
+        qc, kc = (torch.randint(0, 1 << 31, (N, T), generator=g) for _ in range(2))
+        qc[:, 5000:] = torch.where(lone[:, 5000:], kc[:, :-5000], qc[:, 5000:])
+    if kind == "mixed":
+        odd = (at // 1024) % 2 == 1
+        qc = torch.where(odd & (torch.rand((N, T), generator=g) < 0.7), 1000 + at // 3, qc)
+        kc = torch.where(odd, 1000 + at // 3, kc)
+    for dt in (torch.int32, torch.int64):
+        q, k = qc.to(dev, dt), kc.to(dev, dt)
+        want = torch.empty((N, T), dtype=torch.int32, device=dev)
+        _lib.check(_lib.lib().lema_latest_prev_match(
+            q.data_ptr(), k.data_ptr(), q.element_size(), N, T, want.data_ptr(), 4,
+            _lib.stream_of(q)))
+        assert torch.equal(attention.latest_prev_match(q, k, torch.int32), want)
