@@ -73,8 +73,12 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* x, const u
   const uint16_t* const xr[1] = {x + row * D};
   const uint16_t* const dr[1] = {d != nullptr ? d + row * D : nullptr};
   uint16_t* const sr[1] = {d != nullptr ? x_out + row * D : nullptr};
-  norm_rows<1, S>(xr, dr, 1, w, eps, D, lane, sr,
-               [h](int, int e, u32x4 v) { *reinterpret_cast<u32x4*>(h + e) = v; });
+  auto none = [] {};
+  auto put = [h](int, int e, u32x4 v) { *reinterpret_cast<u32x4*>(h + e) = v; };
+  if (d != nullptr)
+    norm_rows<1, S, true>(xr, dr, 1, w, eps, D, lane, sr, none, put);
+  else
+    norm_rows<1, S, false>(xr, dr, 1, w, eps, D, lane, sr, none, put);
 }
 
 // One workgroup (256 threads) per row of V bf16 logits (V % 8 == 0, rows 16-byte aligned):
@@ -178,8 +182,9 @@ extern "C" int lema_rmsnorm_bf16(const void* x, const void* d, const void* w, fl
                "pointers must be 16-byte aligned");
   const int64_t grid = (rows + 3) / 4;
   LEMA_REQUIRE(grid < (int64_t(1) << 31), "too many rows");
-  // rows of up to 2048 (the models' widths) hold 4 steps in registers, longer ones 8
-  auto kernel = D <= 2048 ? rmsnorm_kernel<4> : rmsnorm_kernel<kNormMaxSteps>;
+  // rows of up to 1536 or 2048 (the models' widths) hold 3 or 4 steps in registers, longer
+  // ones 8
+  auto kernel = D <= 1536 ? rmsnorm_kernel<3> : D <= 2048 ? rmsnorm_kernel<4> : rmsnorm_kernel<kNormMaxSteps>;
   kernel<<<dim3(grid), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(d),
       static_cast<const uint16_t*>(w), eps, rows, static_cast<int>(D),

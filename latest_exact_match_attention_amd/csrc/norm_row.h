@@ -23,37 +23,52 @@ __device__ __forceinline__ uint32_t nr_f32_to_bf16(float f) {
   if ((b & 0x7F800000u) == 0x7F800000u && (b & 0x007FFFFFu) != 0) return 0x7FC0u;
   return (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
 }
+// Sum over the wavefront, lanes paired 32, 16, 8, 4, 2 and 1 apart in that order. The last four
+// pairings stay inside a row of 16 lanes and are data-parallel moves (a rotation by 4 brings
+// the value of the lane 4 apart, since lanes 8 apart are equal by then, and so on); as LDS
+// permutes each of them waited for the one before.
+template <int kRor>
+__device__ __forceinline__ float nr_add_ror(float v) {
+  const int x = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + kRor, 0xf, 0xf, false);
+  return v + __int_as_float(x);
+}
 __device__ __forceinline__ float nr_wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  v += __shfl_xor(v, 32);
+  v += __shfl_xor(v, 16);
+  v = nr_add_ror<8>(v);
+  v = nr_add_ror<4>(v);
+  v = nr_add_ror<2>(v);
+  return nr_add_ror<1>(v);
 }
 
 // Up to R rows (`n` of them, n <= R) at once by one wavefront, each exactly as alone: rows r
-// start at x[r] (and d[r], null: no addend); s goes to s_out[r] when d[r] and s_out[r] are
-// given, and h's 8 elements at each offset e to put_h(r, e, h8). Every global read (the rows'
-// x and d and the weight) is issued before the first reduction, so the rows cost one round
-// trip. S (at most kNormMaxSteps) bounds the steps, D <= 512 * S: it sizes the registers that
-// hold the rows.
-template <int R, int S, typename PutH>
+// start at x[r] (and d[r] with kAdd); s goes to s_out[r] when kAdd and s_out[r] is given, and
+// h's 8 elements at each offset e to put_h(r, e, h8). Every global read (the rows' x and d and
+// the weight) is issued before the first reduction, so the rows cost one round trip, and
+// loaded() is called between the two, for reads of the caller's that should be in flight
+// meanwhile. No read is conditional (lanes past the row and rows past n read in-bounds
+// elements that nothing uses), so the compiler knows how many are outstanding and waits for
+// the rows alone. S (at most kNormMaxSteps) bounds the steps, D <= 512 * S: it sizes the
+// registers that hold the rows. x[r] (and d[r]) must be readable for every r < R.
+template <int R, int S, bool kAdd, typename Loaded, typename PutH>
 __device__ __forceinline__ void norm_rows(const uint16_t* const (&x)[R], const uint16_t* const (&d)[R],
                                           int n, const uint16_t* w, float eps, int D, int lane,
-                                          uint16_t* const (&s_out)[R], PutH put_h) {
+                                          uint16_t* const (&s_out)[R], Loaded loaded, PutH put_h) {
   const int steps = D / 512 + (D % 512 ? 1 : 0);
   static_assert(S >= 1 && S <= kNormMaxSteps, "steps of 512 elements");
   u32x4 xv[R][S], dv[R][S], wv[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int e = (s * 64 + lane) * 8;
-    if (s >= steps || e >= D) continue;
+    const int e0 = (s * 64 + lane) * 8;
+    const int e = e0 < D ? e0 : 0;
     wv[s] = *reinterpret_cast<const u32x4*>(w + e);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      if (r >= n) continue;
       xv[r][s] = *reinterpret_cast<const u32x4*>(x[r] + e);
-      if (d[r] != nullptr) dv[r][s] = *reinterpret_cast<const u32x4*>(d[r] + e);
+      if constexpr (kAdd) dv[r][s] = *reinterpret_cast<const u32x4*>(d[r] + e);
     }
   }
+  loaded();
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (r >= n) continue;
@@ -63,7 +78,7 @@ __device__ __forceinline__ void norm_rows(const uint16_t* const (&x)[R], const u
       const int e = (s * 64 + lane) * 8;
       if (s >= steps || e >= D) continue;
       u32x4 v = xv[r][s];
-      if (d[r] != nullptr) {
+      if constexpr (kAdd) {
         uint32_t* pv = reinterpret_cast<uint32_t*>(&v);
         const uint32_t* pd = reinterpret_cast<const uint32_t*>(&dv[r][s]);
 #pragma unroll

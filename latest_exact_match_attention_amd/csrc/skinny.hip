@@ -26,6 +26,8 @@
 // Operand layout of v_mfma_f32_16x16x32_bf16 (checked on the device): lane l holds A row l%16
 // and B column l%16, k = 8 * (l / 16) + j, j < 8; the result's register r of lane l is row
 // 4 * (l / 16) + r, column l % 16.
+#include <type_traits>
+
 #include "lema_internal.h"
 #include "norm_row.h"
 
@@ -37,7 +39,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSkThreads = 512;
 constexpr int kSkWaves = kSkThreads / 64;
-constexpr int kSkUnroll = 4;  // K-steps of 32 with loads in flight per wavefront
+constexpr int kSkShortK = 1536;  // rows of up to this (kShort) or kSkNormSteps * 512 elements
 constexpr int kSkNormSteps = 4;  // a fused pre-norm's rows: up to 4 * 512 elements in registers
 
 // One weight segment of a launch: its blocks cover N output columns of x . w^T with one
@@ -51,8 +53,7 @@ struct SkSegment {
   void* out;           // plain / swiglu: bf16 [M, ldy]; pack: codes
   const uint16_t* res; // plain: optional bf16 [M, ldy] residual, out = bf16(res + bf16(sum))
   int64_t ldy;
-  int32_t N, mode, blocks, code_bytes;
-  int32_t cols;        // output columns per block (set at launch; swiglu: of the gate and of up)
+  int32_t N, mode, code_bytes;
 };
 
 // A product on few blocks leaves CUs idle, and each block's weight read is bound by what its
@@ -78,6 +79,30 @@ struct SkinnyArgs {
   float eps;
 };
 
+// What the kernel gets of it: two cache lines of arguments, the first one all that a plain
+// product needs. The argument lines are cold at every launch, and the weights' loads wait for
+// them (with the four lines of SkinnyArgs every launch took 0.3 to 0.5 us more).
+struct SkDevice {
+  const uint16_t* x;
+  const uint16_t* w;
+  void* out;
+  const uint16_t* add;   // plain: the residual or null; pre-norm: the addend or null
+  uint32_t ldx8, ldw8;   // row strides of x and the weights, in 8 elements
+  int32_t K, N;
+  int64_t ldy;
+  uint32_t flags;        // mode | segments << 2 | code bytes << 4 | columns per block << 8 | M << 16
+  int32_t blocks;        // of the first segment, and of the second
+  const uint16_t* w1;    // the second segment's, or swiglu's up
+  const uint16_t* w2;    // the third segment's: plain, Nv columns
+  void* out1;
+  void* out2;
+  const uint16_t* nw;
+  uint16_t* ns;
+  float eps;
+  int32_t d, T, Nv;
+};
+static_assert(sizeof(SkDevice) == 128, "two cache lines");
+
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
   const uint32_t b = __float_as_uint(f);
   if ((b & 0x7F800000u) == 0x7F800000u && (b & 0x007FFFFFu) != 0) return 0x7FC0u;
@@ -91,73 +116,126 @@ __device__ __forceinline__ bool bf16_nonneg(float z) {
 }
 
 // A block owns `cols` columns: 16 * CT, or 8 for a narrow plain segment (swiglu: 16 columns
-// of the gate and the same 16 of up).
-template <int MT, int CT, bool kNorm>
-__global__ __launch_bounds__(kSkThreads) void skinny_kernel(SkinnyArgs a) {
+// of the gate and the same 16 of up). kNorm: 0 = x as it is, 1 = norm(x), 2 = norm(x + nd).
+//
+// Bound: the block's weight read, by the bytes its CU has in flight. So no load is conditional:
+// lanes without a column or row of their own, and steps past a wavefront's share, read
+// in-bounds elements whose products nothing uses. With a load per branch the compiler waited
+// for every load of a group of 4 steps before its products and issued the next group after
+// them. U is the K-steps of a group; the next group's loads are issued before the current one's
+// products, so a wavefront has one to two groups in flight. With a pre-norm one group is all
+// of its share (6 steps for K of up to 1536, 8 up to 2048), and the weights' loads are issued
+// before the pre-norm's arithmetic and arrive meanwhile.
+//
+// kHalf: a narrow block (8 columns) of at most 8 rows fills the matrix tile's idle quarters with
+// a second K-step: columns and rows 8..15 are the same columns and rows one step on, and the
+// two diagonal quarters of the result are added in the reduction. Half the load instructions
+// (the lanes past the block's columns would repeat others' loads at the same cost).
+//
+// Measured, launches in a graph over weights from HBM, before and now: M = 1, K = 1536,
+// N = 1536 4.60 and 3.57 us, N = 4096 5.49 and 4.71, N = 8192 8.26 and 6.92; K = 4096, N = 1536
+// 6.96 and 5.03; M = 16, N = 8192 10.9 and 8.9.
+template <int MT, int CT, int kNorm, int U, bool kHalf>
+__global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 4 : 2) void skinny_kernel(SkDevice a) {
+  constexpr int kSteps = U == 6 ? kSkShortK / 512 : kSkNormSteps;  // the norm's
+  static_assert(kNorm == 0 || 512 * kSteps <= 32 * kSkWaves * U, "one group of loads");
+  static_assert(!kHalf || (MT == 1 && CT == 1 && kNorm == 0), "a half-filled tile");
   __shared__ float part[kSkWaves][MT * 16][CT * 16 + 1];
   extern __shared__ __align__(16) uint16_t xs[];  // kNorm: the normalised rows, stride K + 8
-  int bid = blockIdx.x, si = 0;
-  while (si + 1 < a.nseg && bid >= a.seg[si].blocks) {
-    bid -= a.seg[si].blocks;
-    ++si;
+  const int M = a.flags >> 16, cols = (a.flags >> 8) & 0xFF, code_bytes = (a.flags >> 4) & 0xF;
+  int mode = a.flags & 3, N = a.N, bid = blockIdx.x;
+  const uint16_t* wbase = a.w;
+  void* dst = a.out;
+  if (((a.flags >> 2) & 3) == 3) {  // q, k and v
+    const bool s1 = bid >= a.blocks, s2 = bid >= 2 * a.blocks;
+    wbase = s2 ? a.w2 : s1 ? a.w1 : wbase;
+    dst = s2 ? a.out2 : s1 ? a.out1 : dst;
+    mode = s2 ? kSkPlain : mode;
+    N = s2 ? a.Nv : N;
+    bid -= s2 ? 2 * a.blocks : s1 ? a.blocks : 0;
   }
-  const SkSegment& sg = a.seg[si];
-  const bool glu = sg.mode == kSkSwiglu;
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int cols = sg.cols;
+  const bool glu = mode == kSkSwiglu;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int64_t ldx = static_cast<int64_t>(a.ldx8) * 8, ldw = static_cast<int64_t>(a.ldw8) * 8;
   const int n0 = bid * cols;
-  const int ksteps = a.K / 32;
+  const int ksteps = a.K / (kHalf ? 64 : 32);
+  constexpr int kStep = kHalf ? 64 : 32;
   const int per = (ksteps + kSkWaves - 1) / kSkWaves;
   const int s0 = wave * per;
   const int s1 = s0 + per < ksteps ? s0 + per : ksteps;
+  const int last = s1 > 0 ? s1 - 1 : 0;  // the step that loads past the share repeat
   const int r16 = l & 15, kg = (l >> 4) * 8;
 
   const uint16_t* wp[CT];
-  bool wok[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
-    const int c = glu ? r16 : 16 * ct + r16;  // column of the block
-    const int n = n0 + c;
-    wok[ct] = c < cols && n < sg.N && (!glu || ct < 2);
-    const uint16_t* base = (glu && ct == 1) ? sg.w2 : sg.w;
-    wp[ct] = base + static_cast<int64_t>(wok[ct] ? n : 0) * a.ldw + kg;
+    // column of the block; a lane past the block's or the segment's columns takes its first
+    const int c = kHalf ? r16 & 7 : glu ? r16 : 16 * ct + r16;
+    const int n = c < cols && n0 + c < N ? n0 + c : n0;
+    const uint16_t* base = (glu && ct == 1) ? a.w1 : wbase;
+    wp[ct] = base + static_cast<int64_t>(n) * ldw + kg + (kHalf ? (r16 >> 3) * 32 : 0);
   }
+  // fragments as four 32-bit words: carried through the loop below as bf16 vectors, the compiler
+  // took them apart into elements and reused half of one fragment's registers for an address
+  typedef u32x4 WFrag[U][CT];
+  typedef u32x4 XFrag[U][MT];
+  auto load_w = [&](WFrag& f, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int at = (s + u < s1 ? s + u : last) * kStep;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) f[u][ct] = *reinterpret_cast<const u32x4*>(wp[ct] + at);
+    }
+  };
+  WFrag wa;
   const uint16_t* xp[MT];
-  bool xok[MT];
-  if constexpr (kNorm) {
+  if constexpr (kNorm != 0) {
     // rows m and m + 8 of x by wavefront m, into LDS (a stride of K + 8 puts the 16 rows a
     // fragment load reads in different banks)
     const int xst = a.K + 8;
-    for (int m = wave; m < a.M; m += 2 * kSkWaves) {
-      const int n = m + kSkWaves < a.M ? 2 : 1;
+    auto rows = [&](int m, auto issue) __attribute__((always_inline)) {
       const uint16_t* xr[2];
       const uint16_t* dr[2];
       uint16_t* sr[2];
+      const int n = m + kSkWaves < M ? 2 : 1;
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
-        const int64_t mr = m + r * kSkWaves < a.M ? m + r * kSkWaves : m;
-        xr[r] = a.x + mr * a.ldx;
-        dr[r] = a.nd != nullptr ? a.nd + mr * a.K : nullptr;
-        sr[r] = blockIdx.x == 0 && a.ns != nullptr ? a.ns + mr * a.K : nullptr;
+        const int64_t mr = m + r * kSkWaves < M ? m + r * kSkWaves : m;
+        xr[r] = a.x + mr * ldx;
+        dr[r] = kNorm == 2 ? a.add + mr * a.K : nullptr;
+        sr[r] = kNorm == 2 && blockIdx.x == 0 ? a.ns + mr * a.K : nullptr;
       }
-      norm_rows<2, kSkNormSteps>(xr, dr, n, a.nw, a.eps, a.K, l, sr, [&](int r, int e, u32x4 h) {
+      auto put = [&](int r, int e, u32x4 h) __attribute__((always_inline)) {
         *reinterpret_cast<u32x4*>(xs + (m + r * kSkWaves) * xst + e) = h;
-      });
-    }
+      };
+      auto loaded = [&]() __attribute__((always_inline)) {
+        if constexpr (decltype(issue)::value) {
+          __builtin_amdgcn_sched_barrier(0);  // the rows' loads first: they are waited for first
+          load_w(wa, s0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      norm_rows<2, kSteps, kNorm == 2>(xr, dr, n, a.nw, a.eps, a.K, l, sr, loaded, put);
+    };
+    if (wave < M)
+      rows(wave, std::true_type{});
+    else
+      load_w(wa, s0);
+    if constexpr (MT == 2)
+      if (wave + 2 * kSkWaves < M) rows(wave + 2 * kSkWaves, std::false_type{});
     __syncthreads();
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int m = 16 * mt + r16;
-      xok[mt] = m < a.M;
-      xp[mt] = xs + (xok[mt] ? m : 0) * xst + kg;
+      xp[mt] = xs + (m < M ? m : 0) * xst + kg;
     }
   } else {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      const int m = 16 * mt + r16;
-      xok[mt] = m < a.M;
-      xp[mt] = a.x + static_cast<int64_t>(xok[mt] ? m : 0) * a.ldx + kg;
+      const int m = kHalf ? r16 & 7 : 16 * mt + r16;
+      xp[mt] = a.x + static_cast<int64_t>(m < M ? m : 0) * ldx + kg + (kHalf ? (r16 >> 3) * 32 : 0);
     }
+    load_w(wa, s0);
   }
 
   f32x4 acc[MT][CT];
@@ -165,26 +243,65 @@ __global__ __launch_bounds__(kSkThreads) void skinny_kernel(SkinnyArgs a) {
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) acc[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bf16x8 zero8 = {};
-  for (int s = s0; s < s1; s += kSkUnroll) {
-    bf16x8 wf[kSkUnroll][CT], xf[kSkUnroll][MT];
+  auto load_x = [&](XFrag& f, int s) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kSkUnroll; ++u) {
-      const bool in = s + u < s1;
+    for (int u = 0; u < U; ++u) {
+      const int at = (s + u < s1 ? s + u : last) * kStep;
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-        wf[u][ct] = (in && wok[ct]) ? *reinterpret_cast<const bf16x8*>(wp[ct] + (s + u) * 32) : zero8;
+      for (int mt = 0; mt < MT; ++mt) f[u][mt] = *reinterpret_cast<const u32x4*>(xp[mt] + at);
+    }
+  };
+  // `end`: the share may end inside the group. Steps past it are left out, with x from memory; with
+  // x from LDS they multiply zeros (both factors, so that a stray infinity adds nothing): a
+  // branch would put each fragment's LDS read behind the product before it
+  auto products = [&](WFrag& w, XFrag& x, int s, bool end) __attribute__((always_inline)) {
+    if (kNorm != 0 && end) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        xf[u][mt] = (in && xok[mt]) ? *reinterpret_cast<const bf16x8*>(xp[mt] + (s + u) * 32) : zero8;
+      for (int u = 0; u < U; ++u) {
+        const bool in = s + u < s1;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) w[u][ct] = in ? w[u][ct] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) x[u][mt] = in ? x[u][mt] : u32x4{0u, 0u, 0u, 0u};
+      }
     }
 #pragma unroll
-    for (int u = 0; u < kSkUnroll; ++u)
+    for (int u = 0; u < U; ++u) {
+      if (kNorm == 0 && end && s + u >= s1) break;  // the same in every lane
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
-          acc[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[u][mt], wf[u][ct], acc[mt][ct], 0, 0, 0);
+          acc[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, x[u][mt]), __builtin_bit_cast(bf16x8, w[u][ct]), acc[mt][ct], 0, 0, 0);
+    }
+  };
+  XFrag xa;
+  load_x(xa, s0);
+  if constexpr (kNorm != 0) {
+    products(wa, xa, s0, true);
+  } else {
+    WFrag wb;
+    XFrag xb;
+    int s = s0;
+    for (;;) {  // two groups a trip, so that neither is copied
+      if (s + U >= s1) {
+        products(wa, xa, s, true);
+        break;
+      }
+      load_w(wb, s + U);
+      load_x(xb, s + U);
+      products(wa, xa, s, false);
+      s += U;
+      if (s + U >= s1) {
+        products(wb, xb, s, true);
+        break;
+      }
+      load_w(wa, s + U);
+      load_x(xa, s + U);
+      products(wb, xb, s, false);
+      s += U;
+    }
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -204,23 +321,65 @@ __global__ __launch_bounds__(kSkThreads) void skinny_kernel(SkinnyArgs a) {
     if (e < kRows * kCols) {
       const int row = e / kCols, col = e - (e / kCols) * kCols;
 #pragma unroll
-      for (int wv = 0; wv < kSkWaves; ++wv) sums[i] += part[wv][row][col];
+      for (int wv = 0; wv < kSkWaves; ++wv) {
+        sums[i] += part[wv][row][col];
+        if constexpr (kHalf) sums[i] += part[wv][(row + 8) & 15][(col + 8) & 15];
+      }
     }
   }
-  if (sg.mode == kSkPlain) {
-    uint16_t* y = static_cast<uint16_t*>(sg.out);
+  if (mode == kSkPlain) {
+    uint16_t* y = static_cast<uint16_t*>(dst);
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int e = threadIdx.x + i * kSkThreads;
       const int row = e / kCols, col = e - (e / kCols) * kCols;
-      if (e < kRows * kCols && row < a.M && col < cols && n0 + col < sg.N) {
-        const int64_t at = static_cast<int64_t>(row) * sg.ldy + n0 + col;
+      if (e < kRows * kCols && row < M && col < cols && n0 + col < N) {
+        const int64_t at = static_cast<int64_t>(row) * a.ldy + n0 + col;
         uint32_t out = f32_to_bf16_bits(sums[i]);
-        if (sg.res != nullptr) out = f32_to_bf16_bits(bf16_bits_to_f32(sg.res[at]) + bf16_bits_to_f32(out));
+        if (kNorm == 0 && a.add != nullptr) out = f32_to_bf16_bits(bf16_bits_to_f32(a.add[at]) + bf16_bits_to_f32(out));
         y[at] = static_cast<uint16_t>(out);
       }
     }
     return;
+  }
+  if constexpr (CT == 2) {
+    if (glu) {  // out = silu(gate) * up, the silu rounded to bf16 first; up is 16 lanes on
+      uint16_t* y = static_cast<uint16_t*>(dst);
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int e = threadIdx.x + i * kSkThreads;
+        const int row = e / kCols, c = e % kCols;
+        const float u = bf16_bits_to_f32(f32_to_bf16_bits(__shfl(sums[i], l | 16)));
+        if (c >= 16 || row >= M || n0 + c >= N) continue;
+        const float g = bf16_bits_to_f32(f32_to_bf16_bits(sums[i]));
+        const float sl = bf16_bits_to_f32(f32_to_bf16_bits(g / (1.0f + expf(-g))));
+        y[static_cast<int64_t>(row) * a.ldy + n0 + c] = static_cast<uint16_t>(f32_to_bf16_bits(sl * u));
+      }
+      return;
+    }
+  }
+  if constexpr (CT == 1) {
+    if (a.d % 8 == 0) {
+      // Heads of whole bytes: a ballot gives a row's 16 bits to its 16 lanes, and the lanes of
+      // columns 0 and 8 write a byte of a code each; the one with the head's last byte also
+      // clears the code's bytes above d. (Through LDS, one thread put a row's bits together
+      // from 16 reads, two barriers later.)
+      const int H = N / a.d;
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int e = threadIdx.x + i * kSkThreads;
+        const uint64_t bal = __ballot(bf16_nonneg(sums[i]));
+        const int row = e / kCols, c = e % kCols, n = n0 + c;
+        if (e >= kRows * kCols || (c & 7) != 0 || row >= M || n >= N) continue;
+        const int h = n / a.d, k = (n - h * a.d) / 8;
+        const int b = row / a.T, t = row - b * a.T;
+        uint8_t* w8 = static_cast<uint8_t*>(dst) + ((static_cast<int64_t>(b) * H + h) * a.T + t) * code_bytes;
+        w8[k] = static_cast<uint8_t>(bal >> l);
+        if (8 * k + 8 == a.d)
+          for (int z = k + 1; z < code_bytes; ++z) w8[z] = 0;
+      }
+      return;
+    }
   }
   __syncthreads();  // every partial is read: the block's sums go to part[0]
 #pragma unroll
@@ -229,74 +388,86 @@ __global__ __launch_bounds__(kSkThreads) void skinny_kernel(SkinnyArgs a) {
     if (e < kRows * kCols) part[0][e / kCols][e - (e / kCols) * kCols] = sums[i];
   }
   __syncthreads();
-  if (glu) {  // out = silu(gate) * up, the silu rounded to bf16 first
-    uint16_t* y = static_cast<uint16_t*>(sg.out);
-    for (int e = threadIdx.x; e < kRows * 16; e += kSkThreads) {
-      const int row = e >> 4, c = e & 15;
-      if (row >= a.M || c >= cols || n0 + c >= sg.N) continue;
-      const float g = bf16_bits_to_f32(f32_to_bf16_bits(part[0][row][c]));
-      const float u = bf16_bits_to_f32(f32_to_bf16_bits(part[0][row][16 + c]));
-      const float sl = bf16_bits_to_f32(f32_to_bf16_bits(g / (1.0f + expf(-g))));
-      y[static_cast<int64_t>(row) * sg.ldy + n0 + c] = static_cast<uint16_t>(f32_to_bf16_bits(sl * u));
-    }
-    return;
-  }
-  // the heads this block's columns [n0, n0 + cols) touch; a head split over blocks gets its
-  // byte-aligned bit range written by each (d is a multiple of 8 then, checked on the host),
-  // the block with its last bit also clearing the code's bytes above d
-  const int H = sg.N / a.d;
+  // whole heads of other widths
+  const int H = N / a.d;
   const int h0 = n0 / a.d;
   const int h1 = min((n0 + cols - 1) / a.d, H - 1);
   const int nh = h1 - h0 + 1;
   for (int e = threadIdx.x; e < kRows * nh; e += kSkThreads) {
     const int row = e / nh, h = h0 + (e - (e / nh) * nh);
-    if (row >= a.M) continue;
+    if (row >= M) continue;
     const int c_lo = max(n0, h * a.d), c_hi = min(n0 + cols, (h + 1) * a.d);
     uint64_t code = 0;
     for (int n = c_lo; n < c_hi; ++n)
       if (bf16_nonneg(part[0][row][n - n0])) code |= uint64_t(1) << (n - h * a.d);
     const int64_t b = row / a.T, t = row - (row / a.T) * a.T;
     const int64_t at = (b * H + h) * a.T + t;
-    const int j_lo = c_lo - h * a.d, j_hi = c_hi - h * a.d;  // bits [j_lo, j_hi) of the code
-    if (j_lo == 0 && j_hi == a.d) {
-      if (sg.code_bytes == 4)
-        static_cast<uint32_t*>(sg.out)[at] = static_cast<uint32_t>(code);
-      else
-        static_cast<uint64_t*>(sg.out)[at] = code;
-    } else {
-      uint8_t* w8 = static_cast<uint8_t*>(sg.out) + at * sg.code_bytes;
-      for (int k = j_lo / 8; k < j_hi / 8; ++k) w8[k] = static_cast<uint8_t>(code >> (8 * k));
-      if (j_hi == a.d)
-        for (int k = a.d / 8; k < sg.code_bytes; ++k) w8[k] = 0;
-    }
+    if (code_bytes == 4)
+      static_cast<uint32_t*>(dst)[at] = static_cast<uint32_t>(code);
+    else
+      static_cast<uint64_t*>(dst)[at] = code;
   }
 }
 
 template <int CT>
 int launch_skinny(SkinnyArgs& a, hipStream_t st) {
+  bool all_plain = true;
+  for (int j = 0; j < a.nseg; ++j) all_plain = all_plain && a.seg[j].mode == kSkPlain;
+  const SkSegment& s0 = a.seg[0];
+  const bool narrow = CT == 1 && all_plain && s0.N <= kNarrowMaxN;
+  const int cols = s0.mode == kSkSwiglu ? 16 : narrow ? kNarrowCols : 16 * CT;
   int blocks = 0;
-  for (int i = 0; i < a.nseg; ++i) {
-    SkSegment& sg = a.seg[i];
-    bool all_plain = true;
-    for (int j = 0; j < a.nseg; ++j) all_plain = all_plain && a.seg[j].mode == kSkPlain;
-    sg.cols = sg.mode == kSkSwiglu ? 16
-              : CT == 1 && all_plain && sg.N <= kNarrowMaxN ? kNarrowCols
-                                                           : 16 * CT;
-    sg.blocks = (sg.N + sg.cols - 1) / sg.cols;
-    blocks += sg.blocks;
-  }
+  for (int i = 0; i < a.nseg; ++i) blocks += (a.seg[i].N + cols - 1) / cols;
+  SkDevice g{};
+  g.x = a.x;
+  g.w = s0.w;
+  g.out = s0.out;
+  g.add = a.nw != nullptr ? a.nd : s0.res;
+  // the stride of a single row is never used
+  g.ldx8 = static_cast<uint32_t>((a.M > 1 ? a.ldx : a.K) / 8);
+  g.ldw8 = static_cast<uint32_t>(a.ldw / 8);
+  g.K = a.K;
+  g.N = s0.N;
+  g.ldy = a.nseg == 3 ? a.seg[2].ldy : s0.ldy;
+  g.flags = static_cast<uint32_t>(s0.mode) | static_cast<uint32_t>(a.nseg) << 2 |
+            static_cast<uint32_t>(s0.code_bytes) << 4 | static_cast<uint32_t>(cols) << 8 |
+            static_cast<uint32_t>(a.M) << 16;
+  g.blocks = (s0.N + cols - 1) / cols;
+  g.w1 = a.nseg == 3 ? a.seg[1].w : s0.w2;
+  g.w2 = a.seg[2].w;
+  g.out1 = a.seg[1].out;
+  g.out2 = a.seg[2].out;
+  g.nw = a.nw;
+  g.ns = a.ns;
+  g.eps = a.eps;
+  g.d = a.d;
+  g.T = a.T;
+  g.Nv = a.seg[2].N;
   const dim3 grid(blocks), block(kSkThreads);
+  const size_t lds = a.nw != nullptr ? static_cast<size_t>(a.M) * (a.K + 8) * sizeof(uint16_t) : 0;
+  void (*kernel)(SkDevice) = nullptr;
   if (a.nw != nullptr) {  // the normalised rows in LDS (checked to fit by the entry point)
-    const size_t lds = static_cast<size_t>(a.M) * (a.K + 8) * sizeof(uint16_t);
-    if (a.M <= 16)
-      skinny_kernel<1, CT, true><<<grid, block, lds, st>>>(a);
+    auto pick = [&](auto mt) {
+      constexpr int MT = decltype(mt)::value;
+      return a.nd != nullptr ? (a.K <= kSkShortK ? skinny_kernel<MT, CT, 2, 6, false> : skinny_kernel<MT, CT, 2, 8, false>)
+                             : (a.K <= kSkShortK ? skinny_kernel<MT, CT, 1, 6, false> : skinny_kernel<MT, CT, 1, 8, false>);
+    };
+    kernel = a.M <= 16 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
+  } else if constexpr (CT == 1) {
+    // K-steps per group: the larger one unless it divides a wavefront's share worse
+    const int per = (a.K / 32 + kSkWaves - 1) / kSkWaves;
+    const int half = (a.K / 64 + kSkWaves - 1) / kSkWaves;
+    auto waste = [](int share, int u) { return (share + u - 1) / u * u - share; };
+    if (narrow && a.M <= 8 && a.K % 64 == 0)
+      kernel = waste(half, 4) <= waste(half, 3) ? skinny_kernel<1, 1, 0, 4, true> : skinny_kernel<1, 1, 0, 3, true>;
+    else if (waste(per, 6) <= waste(per, 4))
+      kernel = a.M <= 16 ? skinny_kernel<1, 1, 0, 6, false> : skinny_kernel<2, 1, 0, 6, false>;
     else
-      skinny_kernel<2, CT, true><<<grid, block, lds, st>>>(a);
-  } else if (a.M <= 16) {
-    skinny_kernel<1, CT, false><<<grid, block, 0, st>>>(a);
+      kernel = a.M <= 16 ? skinny_kernel<1, 1, 0, 4, false> : skinny_kernel<2, 1, 0, 4, false>;
   } else {
-    skinny_kernel<2, CT, false><<<grid, block, 0, st>>>(a);
+    kernel = a.M <= 16 ? skinny_kernel<1, CT, 0, 4, false> : skinny_kernel<2, CT, 0, 4, false>;
   }
+  kernel<<<grid, block, lds, st>>>(g);
   return launch_status("skinny_kernel");
 }
 
@@ -315,6 +486,7 @@ int check_skinny(const void* x, int64_t ldx, int64_t ldw, int64_t M, int64_t K) 
                (long long)K);
   LEMA_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0,
                "row strides must be >= K and multiples of 8");
+  LEMA_REQUIRE((M == 1 || ldx < (int64_t(1) << 34)) && ldw < (int64_t(1) << 34), "row strides past 2^34 elements");
   LEMA_REQUIRE(x != nullptr && aligned(x, 16), "x must be a 16-byte aligned device pointer");
   return LEMA_OK;
 }
@@ -356,7 +528,7 @@ extern "C" int lema_skinny_gemm_bf16(const void* x, int64_t ldx, const void* w, 
   a.K = static_cast<int32_t>(K);
   a.nseg = 1;
   a.seg[0] = SkSegment{static_cast<const uint16_t*>(w), nullptr, y, nullptr, ldy,
-                       static_cast<int32_t>(N), kSkPlain, 0, 0};
+                       static_cast<int32_t>(N), kSkPlain, 0};
   return launch_ct(a, 1, static_cast<hipStream_t>(stream));
 }
 
@@ -375,8 +547,7 @@ extern "C" int lema_skinny_gemm_add_bf16(const void* x, int64_t ldx, const void*
   a.K = static_cast<int32_t>(K);
   a.nseg = 1;
   a.seg[0] = SkSegment{static_cast<const uint16_t*>(w), nullptr, y,
-                       static_cast<const uint16_t*>(r), ldy, static_cast<int32_t>(N), kSkPlain, 0,
-                       0};
+                       static_cast<const uint16_t*>(r), ldy, static_cast<int32_t>(N), kSkPlain, 0};
   return launch_ct(a, 1, static_cast<hipStream_t>(stream));
 }
 
@@ -404,7 +575,7 @@ extern "C" int lema_skinny_pack_bf16(const void* x, int64_t ldx, const void* w, 
   a.T = static_cast<int32_t>(T);
   a.nseg = 1;
   a.seg[0] = SkSegment{static_cast<const uint16_t*>(w), nullptr, codes, nullptr, 0,
-                       static_cast<int32_t>(N), kSkPack, 0, code_bytes};
+                       static_cast<int32_t>(N), kSkPack, code_bytes};
   return launch_ct(a, ct, static_cast<hipStream_t>(stream));
 }
 
@@ -438,11 +609,11 @@ int qkv_args(SkinnyArgs& a, int& ct, const void* x, int64_t ldx, const void* wq,
   a.T = static_cast<int32_t>(T);
   a.nseg = 3;
   a.seg[0] = SkSegment{static_cast<const uint16_t*>(wq), nullptr, qcodes, nullptr, 0,
-                       static_cast<int32_t>(Nqk), kSkPack, 0, code_bytes};
+                       static_cast<int32_t>(Nqk), kSkPack, code_bytes};
   a.seg[1] = SkSegment{static_cast<const uint16_t*>(wk), nullptr, kcodes, nullptr, 0,
-                       static_cast<int32_t>(Nqk), kSkPack, 0, code_bytes};
+                       static_cast<int32_t>(Nqk), kSkPack, code_bytes};
   a.seg[2] = SkSegment{static_cast<const uint16_t*>(wv), nullptr, v, nullptr, Nv,
-                       static_cast<int32_t>(Nv), kSkPlain, 0, 0};
+                       static_cast<int32_t>(Nv), kSkPlain, 0};
   return LEMA_OK;
 }
 
@@ -509,7 +680,7 @@ extern "C" int lema_skinny_swiglu_bf16(const void* x, int64_t ldx, const void* w
   a.K = static_cast<int32_t>(K);
   a.nseg = 1;
   a.seg[0] = SkSegment{static_cast<const uint16_t*>(wg), static_cast<const uint16_t*>(wu), out,
-                       nullptr, N, static_cast<int32_t>(N), kSkSwiglu, 0, 0};
+                       nullptr, N, static_cast<int32_t>(N), kSkSwiglu, 0};
   return launch_ct(a, 2, static_cast<hipStream_t>(stream));
 }
 
@@ -540,7 +711,7 @@ extern "C" int lema_skinny_norm_swiglu_bf16(const void* x, const void* d, const 
   a.K = static_cast<int32_t>(K);
   a.nseg = 1;
   a.seg[0] = SkSegment{static_cast<const uint16_t*>(wg), static_cast<const uint16_t*>(wu), out,
-                       nullptr, N, static_cast<int32_t>(N), kSkSwiglu, 0, 0};
+                       nullptr, N, static_cast<int32_t>(N), kSkSwiglu, 0};
   a.nd = static_cast<const uint16_t*>(d);
   a.nw = static_cast<const uint16_t*>(nw);
   a.ns = static_cast<uint16_t*>(x_out);

@@ -1,0 +1,71 @@
+"""The skinny products where their load groups, tile halves and epilogues can go wrong: K shares
+that end inside a group, wavefronts without a share, up to 8 and more rows (a half-filled tile
+holds a second K-step up to 8), infinities past a share's end, heads split over blocks at every
+byte. Needs a GPU."""
+import pytest
+import torch
+
+from latest_exact_match_attention_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch.device("cuda", 0)
+
+
+def _product(x, w):
+    M, K = x.shape
+    y = torch.empty((M, w.shape[0]), dtype=x.dtype, device=x.device)
+    _lib.check(_lib.lib().lema_skinny_gemm_bf16(
+        x.data_ptr(), K, w.data_ptr(), K, y.data_ptr(), w.shape[0], M, w.shape[0], K,
+        _lib.stream_of(x)))
+    return y
+
+
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("N", [5, 24, 2048, 2056])
+@pytest.mark.parametrize("K", [32, 64, 96, 448, 768, 1536, 1568, 1792, 3072, 4096, 6400])
+def test_shares(dev, M, N, K):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), device=dev, generator=g).to(torch.bfloat16)
+    w = (torch.randn((N, K), device=dev, generator=g) * K ** -0.5).to(torch.bfloat16)
+    ref = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    # one rounding to bf16, and fp32 sums of K products
+    bound = 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * size
+    assert float(((_product(x, w).double() - ref).abs() - bound).max()) <= 0.0
+
+
+def test_an_infinity_stays_in_its_products(dev):
+    """An infinity in the last column of x or a weight touches its own row or column alone."""
+    for K in (1536, 1792, 2048):
+        x = torch.ones((3, K), device=dev, dtype=torch.bfloat16)
+        w = torch.ones((64, K), device=dev, dtype=torch.bfloat16)
+        x[1, K - 1] = float("inf")
+        w[5, K - 1] = float("-inf")
+        y = _product(x, w).float()
+        want = x.float() @ w.float().T
+        assert torch.equal(torch.isnan(y), torch.isnan(want))
+        assert torch.equal(y.nan_to_num(1.0, 2.0, 3.0), want.nan_to_num(1.0, 2.0, 3.0))
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 31])
+@pytest.mark.parametrize("d,cb", [(8, 4), (24, 4), (24, 8), (32, 4), (40, 8), (56, 8), (64, 8), (4, 4), (12, 8)])
+def test_code_bytes(dev, M, d, cb):
+    """Every byte of a code, those above d cleared, for heads that blocks split and hold."""
+    H, K = 6, 256
+    g = torch.Generator(device=dev).manual_seed(d + M)
+    # integer products: the signs are exact
+    x = torch.randint(-3, 4, (M, K), device=dev, generator=g).to(torch.bfloat16)
+    w = torch.randint(-3, 4, (H * d, K), device=dev, generator=g).to(torch.bfloat16)
+    z = x.double() @ w.double().T
+    want = ((z.view(M, H, d) >= 0).long() << torch.arange(d, device=dev)).sum(-1).t()
+    codes = torch.full((H, M), -1, dtype=torch.int32 if cb == 4 else torch.int64, device=dev)
+    _lib.check(_lib.lib().lema_skinny_pack_bf16(x.data_ptr(), K, w.data_ptr(), K, M, H * d, K, d, M,
+                                                codes.data_ptr(), cb, _lib.stream_of(x)))
+    got = codes.long() & 0xFFFFFFFF if cb == 4 else codes
+    assert torch.equal(got, want)
