@@ -94,6 +94,20 @@ int lema_hard_ws(const void* qc, const void* kc, int32_t code_bytes, const void*
                  int32_t miss, void* src, int32_t src_bytes, void* workspace,
                  int64_t workspace_bytes, void* stream);
 
+/* lema_hard from the projected queries and keys: both packed as by lema_pack_codes (code_bytes
+ * 4 for D <= 32, else 8) in one launch when their strides agree, then lema_hard_ws on the
+ * codes. Replaces lema_hard(q, k, v) without a store, code/lema/attention.py:135-158.
+ *   q, k       [B, H, T, D] of `z_dtype`, element strides, last dim contiguous
+ *   workspace  256-byte aligned device memory of lema_hard_z_workspace_bytes(B*H, T,
+ *              code_bytes) bytes: the codes, and lema_hard_ws's scratch */
+int64_t lema_hard_z_workspace_bytes(int64_t N, int64_t T, int32_t code_bytes);
+int lema_hard_z(const void* q, const void* k, int32_t z_dtype, int32_t D, int64_t q_sb, int64_t q_sh,
+                int64_t q_st, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v, int32_t dtype,
+                int64_t B, int64_t H, int64_t T, int64_t dv, int64_t v_sb, int64_t v_sh,
+                int64_t v_st, void* y, int64_t y_sb, int64_t y_sh, int64_t y_st, int32_t miss,
+                void* src, int32_t src_bytes, void* workspace, int64_t workspace_bytes,
+                void* stream);
+
 /* The gather alone, for given indices: y = v[src] (miss per `miss`).
  * Replaces code/lema/attention.py:157-158. Shapes and strides as in lema_hard;
  * src is contiguous [B*H, T] of src_bytes, every entry in [-1, T).                      */

@@ -45,6 +45,10 @@ PROTOTYPES = {
                       _i64, _i64, _i64, _i32, _p, _i32, _p, _i64, _p], ctypes.c_int),
     "lema_gather": ([_p, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i32, _p, _i64,
                      _i64, _i64, _i32, _p], ctypes.c_int),
+    "lema_hard_z_workspace_bytes": ([_i64, _i64, _i32], ctypes.c_int64),
+    "lema_hard_z": ([_p, _p, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i32, _i64, _i64,
+                     _i64, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i32, _p, _i32, _p, _i64,
+                     _p], ctypes.c_int),
     "lema_gather_grad": ([_p, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p, _p],
                          ctypes.c_int),
     "lema_store_exchange": ([_p, _i64, _i64, _p, _p, _i32, _p, _p, _i64, _i64, _i64, _p, _p, _p],

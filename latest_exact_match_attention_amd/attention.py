@@ -192,6 +192,40 @@ def gather_values(v: torch.Tensor, src: torch.Tensor, miss: str = "dense") -> to
     return y
 
 
+def _one_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether lema_hard_z takes these as they are: everything it checks holds, nothing has to
+    be copied first. Any other call (errors among them) goes the way of pack_codes and
+    lema_from_codes."""
+    D = q.shape[-1]
+    return (q.dim() == 4 and q.shape == k.shape and q.dtype == k.dtype and v.dim() == 4
+            and v.shape[:3] == q.shape[:3] and 1 <= D <= 64 and q.is_cuda
+            and q.device == k.device == v.device and q.dtype in _lib.DTYPE_CODE
+            and v.dtype in _lib.DTYPE_CODE and v.numel() > 0
+            and (q.stride(3) == k.stride(3) == 1 or D == 1)
+            and (v.stride(3) == 1 or v.shape[3] == 1))
+
+
+def _hard_z(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+            want_src: bool) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """_hard_forward from pre-activations, in one library call."""
+    L = _lib.lib()
+    B, H, T, dv = v.shape
+    D = q.shape[3]
+    y = torch.empty_like(v)
+    if y.stride(3) != 1 and dv > 1:
+        y = torch.empty(v.shape, dtype=v.dtype, device=v.device)
+    src = torch.empty((B, H, T), dtype=torch.int32, device=v.device) if want_src else None
+    n = L.lema_hard_z_workspace_bytes(B * H, T, 4 if D <= 32 else 8)
+    ws = torch.empty(n, dtype=torch.uint8, device=v.device)
+    qs, ks, vs, ys = q.stride(), k.stride(), v.stride(), y.stride()
+    _lib.check(L.lema_hard_z(
+        q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[q.dtype], D, qs[0], qs[1], qs[2], ks[0], ks[1],
+        ks[2], v.data_ptr(), _lib.DTYPE_CODE[v.dtype], B, H, T, dv, vs[0], vs[1], vs[2],
+        y.data_ptr(), ys[0], ys[1], ys[2], _lib.MISS_DENSE,
+        src.data_ptr() if src is not None else None, 4, ws.data_ptr(), n, _lib.stream_of(v)))
+    return y, src
+
+
 def _plain_grad(gy: torch.Tensor) -> bool:
     """Whether a backward may hand gy to the kernel: an ordinary device tensor whose own
     gradient nobody asks for. A graph of the backward (create_graph), forward mode, batched
@@ -211,7 +245,9 @@ class _LemaGather(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qc, kc, v):
-        y, src = _hard_forward(qc, kc, v, want_src=True)
+        """qc, kc: the codes, or the pre-activations of a call that _one_call takes."""
+        run = _hard_z if qc.is_floating_point() else _hard_forward
+        y, src = run(qc, kc, v, want_src=True)
         ctx.save_for_backward(src)
         ctx.v_shape = v.shape
         return y
@@ -247,6 +283,10 @@ def lema_hard(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, store=None) -> 
     B, H, T, D = q.shape
     if D > 64:
         raise ValueError(f"d_qk {D} > 64 cannot pack into a uint64")
+    if store is None and _one_call(q, k, v):
+        if v.requires_grad and torch.is_grad_enabled():
+            return _LemaGather.apply(q.detach(), k.detach(), v)
+        return _hard_z(q, k, v, want_src=False)[0]
     with torch.no_grad():
         ct = code_dtype_for(D)
         qc, kc = pack_codes(q, ct), pack_codes(k, ct)

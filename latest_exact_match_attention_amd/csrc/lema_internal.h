@@ -69,6 +69,11 @@ struct FastDiv {
   }
 };
 
+// pack.hip: sign-pack z, and z2 of the same layout when given, in one launch (arguments checked).
+int pack_launch(const void* z, void* codes, const void* z2, void* codes2, int32_t dtype, int64_t B, int64_t H,
+                int64_t T, int32_t D, int64_t z_sb, int64_t z_sh, int64_t z_st, int32_t code_bytes,
+                hipStream_t st);
+
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs, each with its own
 // 4 MB L2; kernels map blockIdx so that work sharing data lands on one XCD.
 constexpr int kNumXcd = 8;

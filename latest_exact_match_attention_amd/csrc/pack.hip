@@ -33,6 +33,8 @@ __device__ __forceinline__ bool nonneg(const void* z, int64_t e) {
 struct DenseArgs {
   const void* z;
   void* codes;
+  const void* z2;       // workgroups of blockIdx.y = 1: another tensor of the same layout (the
+  void* codes2;         // keys beside the queries), packed in the same launch
   int64_t R;            // rows
   int64_t E1, E2;       // extents of the two inner memory-order dims
   int64_t os0, os1, os2;  // output strides (codes) of the memory-order dims
@@ -144,6 +146,10 @@ __device__ __forceinline__ int64_t out_index(const DenseArgs& a, int64_t m) {
 
 template <int DTYPE, typename CodeT>
 __global__ __launch_bounds__(kPackThreads) void pack_dense_kernel(DenseArgs a) {
+  if (blockIdx.y) {
+    a.z = a.z2;
+    a.codes = a.codes2;
+  }
   __shared__ uint64_t words[kPackThreads / 64][64 + 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t m0 = (static_cast<int64_t>(blockIdx.x) * (kPackThreads / 64) + w) * 64;
@@ -163,6 +169,10 @@ __global__ __launch_bounds__(kPackThreads) void pack_dense_kernel(DenseArgs a) {
 // 6.0 with 16, 10.0 with 32; a read of the same bytes alone takes 33.3 and 4.4 us).
 template <int DTYPE, typename CodeT, int G>
 __global__ __launch_bounds__(kPackThreads) void pack_tile_kernel(DenseArgs a) {
+  if (blockIdx.y) {
+    a.z = a.z2;
+    a.codes = a.codes2;
+  }
   __shared__ uint64_t words[kPackThreads / 64][64 + 1];
   __shared__ CodeT tile[G][64 + 1];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -182,6 +192,8 @@ __global__ __launch_bounds__(kPackThreads) void pack_tile_kernel(DenseArgs a) {
 struct StridedArgs {
   const void* z;
   void* codes;
+  const void* z2;
+  void* codes2;
   int64_t B, H, T;
   int64_t sb, sh, st;
   int32_t D;
@@ -189,6 +201,10 @@ struct StridedArgs {
 
 template <int DTYPE, typename CodeT>
 __global__ __launch_bounds__(kPackThreads) void pack_strided_kernel(StridedArgs a) {
+  if (blockIdx.y) {
+    a.z = a.z2;
+    a.codes = a.codes2;
+  }
   const int64_t r = static_cast<int64_t>(blockIdx.x) * kPackThreads + threadIdx.x;
   if (r >= a.B * a.H * a.T) return;
   const int64_t t = r % a.T;
@@ -206,9 +222,9 @@ int launch_tile(int32_t dtype, const DenseArgs& a, hipStream_t st) {
   const int64_t grid = (a.R + G * 64 - 1) / (G * 64);
   LEMA_REQUIRE(grid < (int64_t(1) << 31), "too many rows to pack");
   switch (dtype) {
-    case LEMA_F32: pack_tile_kernel<LEMA_F32, CodeT, G><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
-    case LEMA_F16: pack_tile_kernel<LEMA_F16, CodeT, G><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
-    default: pack_tile_kernel<LEMA_BF16, CodeT, G><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
+    case LEMA_F32: pack_tile_kernel<LEMA_F32, CodeT, G><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
+    case LEMA_F16: pack_tile_kernel<LEMA_F16, CodeT, G><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
+    default: pack_tile_kernel<LEMA_BF16, CodeT, G><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
   }
   return launch_status("pack_tile_kernel");
 }
@@ -221,9 +237,9 @@ int launch_dense(int32_t dtype, const DenseArgs& a, hipStream_t st) {
   const int64_t grid = (a.R + kPackThreads - 1) / kPackThreads;
   LEMA_REQUIRE(grid < (int64_t(1) << 31), "too many rows to pack");
   switch (dtype) {
-    case LEMA_F32: pack_dense_kernel<LEMA_F32, CodeT><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
-    case LEMA_F16: pack_dense_kernel<LEMA_F16, CodeT><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
-    default: pack_dense_kernel<LEMA_BF16, CodeT><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
+    case LEMA_F32: pack_dense_kernel<LEMA_F32, CodeT><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
+    case LEMA_F16: pack_dense_kernel<LEMA_F16, CodeT><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
+    default: pack_dense_kernel<LEMA_BF16, CodeT><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
   }
   return launch_status("pack_dense_kernel");
 }
@@ -233,14 +249,48 @@ int launch_strided(int32_t dtype, const StridedArgs& a, hipStream_t st) {
   const int64_t grid = (a.B * a.H * a.T + kPackThreads - 1) / kPackThreads;
   LEMA_REQUIRE(grid < (int64_t(1) << 31), "too many rows to pack");
   switch (dtype) {
-    case LEMA_F32: pack_strided_kernel<LEMA_F32, CodeT><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
-    case LEMA_F16: pack_strided_kernel<LEMA_F16, CodeT><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
-    default: pack_strided_kernel<LEMA_BF16, CodeT><<<dim3(grid), dim3(kPackThreads), 0, st>>>(a); break;
+    case LEMA_F32: pack_strided_kernel<LEMA_F32, CodeT><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
+    case LEMA_F16: pack_strided_kernel<LEMA_F16, CodeT><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
+    default: pack_strided_kernel<LEMA_BF16, CodeT><<<dim3(grid, a.z2 != nullptr ? 2 : 1), dim3(kPackThreads), 0, st>>>(a); break;
   }
   return launch_status("pack_strided_kernel");
 }
 
 }  // namespace
+
+// Packs z (and z2, another tensor of the same layout, when given) in one launch; the layout has
+// been checked.
+int pack_launch(const void* z, void* codes, const void* z2, void* codes2, int32_t dtype, int64_t B, int64_t H,
+                int64_t T, int32_t D, int64_t z_sb, int64_t z_sh, int64_t z_st, int32_t code_bytes,
+                hipStream_t st) {
+  const int64_t R = B * H * T;
+  // Are the rows one packed array? Drop unit dims, order the rest by stride (outermost
+  // first) and check that each stride is the product of the inner extents times D.
+  struct Dim { int64_t e, s, os; };
+  Dim dims[3] = {{B, z_sb, H * T}, {H, z_sh, T}, {T, z_st, 1}};
+  Dim kept[3];
+  int nk = 0;
+  for (const Dim& d : dims)
+    if (d.e > 1) kept[nk++] = d;
+  for (int i = 0; i < nk; ++i)
+    for (int j = i + 1; j < nk; ++j)
+      if (kept[j].s > kept[i].s) { Dim x = kept[i]; kept[i] = kept[j]; kept[j] = x; }
+  bool dense = true;
+  int64_t need = D;
+  for (int i = nk - 1; i >= 0; --i) {
+    dense = dense && kept[i].s == need;
+    need *= kept[i].e;
+  }
+  if (dense && aligned(z, 16) && (z2 == nullptr || aligned(z2, 16))) {
+    Dim full[3] = {{1, 0, 0}, {1, 0, 0}, {1, 0, 0}};
+    for (int i = 0; i < nk; ++i) full[3 - nk + i] = kept[i];
+    DenseArgs a{z, codes, z2, codes2, R, full[1].e, full[2].e, full[0].os, full[1].os, full[2].os, D};
+    return code_bytes == 4 ? launch_dense<uint32_t>(dtype, a, st) : launch_dense<uint64_t>(dtype, a, st);
+  }
+  StridedArgs a{z, codes, z2, codes2, B, H, T, z_sb, z_sh, z_st, D};
+  return code_bytes == 4 ? launch_strided<uint32_t>(dtype, a, st) : launch_strided<uint64_t>(dtype, a, st);
+}
+
 }  // namespace lema
 
 using namespace lema;
@@ -259,31 +309,6 @@ extern "C" int lema_pack_codes(const void* z, int32_t dtype, int64_t B, int64_t 
   if (R == 0) return LEMA_OK;
   LEMA_REQUIRE(z != nullptr && codes != nullptr, "null pointer");
   LEMA_REQUIRE(aligned(z, es) && aligned(codes, code_bytes), "misaligned pointer");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-
-  // Are the rows one packed array? Drop unit dims, order the rest by stride (outermost
-  // first) and check that each stride is the product of the inner extents times D.
-  struct Dim { int64_t e, s, os; };
-  Dim dims[3] = {{B, z_sb, H * T}, {H, z_sh, T}, {T, z_st, 1}};
-  Dim kept[3];
-  int nk = 0;
-  for (const Dim& d : dims)
-    if (d.e > 1) kept[nk++] = d;
-  for (int i = 0; i < nk; ++i)
-    for (int j = i + 1; j < nk; ++j)
-      if (kept[j].s > kept[i].s) { Dim x = kept[i]; kept[i] = kept[j]; kept[j] = x; }
-  bool dense = true;
-  int64_t need = D;
-  for (int i = nk - 1; i >= 0; --i) {
-    dense = dense && kept[i].s == need;
-    need *= kept[i].e;
-  }
-  if (dense && aligned(z, 16)) {
-    Dim full[3] = {{1, 0, 0}, {1, 0, 0}, {1, 0, 0}};
-    for (int i = 0; i < nk; ++i) full[3 - nk + i] = kept[i];
-    DenseArgs a{z, codes, R, full[1].e, full[2].e, full[0].os, full[1].os, full[2].os, D};
-    return code_bytes == 4 ? launch_dense<uint32_t>(dtype, a, st) : launch_dense<uint64_t>(dtype, a, st);
-  }
-  StridedArgs a{z, codes, B, H, T, z_sb, z_sh, z_st, D};
-  return code_bytes == 4 ? launch_strided<uint32_t>(dtype, a, st) : launch_strided<uint64_t>(dtype, a, st);
+  return pack_launch(z, codes, nullptr, nullptr, dtype, B, H, T, D, z_sb, z_sh, z_st, code_bytes,
+                     static_cast<hipStream_t>(stream));
 }

@@ -664,6 +664,51 @@ extern "C" int lema_hard_ws(const void* qc, const void* kc, int32_t code_bytes, 
               miss, src, src_bytes, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
+// Scratch of lema_hard_z: the query codes, the key codes, then lema_hard_ws's workspace.
+namespace {
+int64_t z_codes_bytes(int64_t N, int64_t T, int32_t code_bytes) {
+  return (N * T * code_bytes + 255) / 256 * 256;
+}
+}  // namespace
+
+extern "C" int64_t lema_hard_z_workspace_bytes(int64_t N, int64_t T, int32_t code_bytes) {
+  return 2 * z_codes_bytes(N, T, code_bytes) + summary_layout(N, T).bytes;
+}
+
+extern "C" int lema_hard_z(const void* q, const void* k, int32_t z_dtype, int32_t D, int64_t q_sb,
+                           int64_t q_sh, int64_t q_st, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                           const void* v, int32_t dtype, int64_t B, int64_t H, int64_t T, int64_t dv,
+                           int64_t v_sb, int64_t v_sh, int64_t v_st, void* y, int64_t y_sb,
+                           int64_t y_sh, int64_t y_st, int32_t miss, void* src, int32_t src_bytes,
+                           void* workspace, int64_t workspace_bytes, void* stream) {
+  clear_error();
+  const int es = dtype_size(z_dtype);
+  LEMA_REQUIRE(es > 0, "unknown query/key dtype %d", z_dtype);
+  LEMA_REQUIRE(D >= 1 && D <= 64, "d_qk %d > 64 cannot pack into a uint64", D);
+  LEMA_REQUIRE(B >= 0 && H >= 0 && T >= 0, "negative shape");
+  if (B * H * T == 0) return LEMA_OK;
+  const int32_t cb = D <= 32 ? 4 : 8;
+  LEMA_REQUIRE(q != nullptr && k != nullptr && aligned(q, es) && aligned(k, es), "bad query or key pointer");
+  LEMA_REQUIRE(workspace != nullptr && aligned(workspace, 256) &&
+                   workspace_bytes >= lema_hard_z_workspace_bytes(B * H, T, cb),
+               "workspace of %lld bytes (256-byte aligned) needed, got %lld",
+               (long long)lema_hard_z_workspace_bytes(B * H, T, cb), (long long)workspace_bytes);
+  uint8_t* qc = static_cast<uint8_t*>(workspace);
+  uint8_t* kc = qc + z_codes_bytes(B * H, T, cb);
+  uint8_t* ws = kc + z_codes_bytes(B * H, T, cb);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  // one launch where both take the same path (a 16-byte aligned packed array, or not)
+  if (q_sb == k_sb && q_sh == k_sh && q_st == k_st && aligned(q, 16) == aligned(k, 16)) {
+    if (int rc = pack_launch(q, qc, k, kc, z_dtype, B, H, T, D, q_sb, q_sh, q_st, cb, st)) return rc;
+  } else {
+    if (int rc = pack_launch(q, qc, nullptr, nullptr, z_dtype, B, H, T, D, q_sb, q_sh, q_st, cb, st)) return rc;
+    if (int rc = pack_launch(k, kc, nullptr, nullptr, z_dtype, B, H, T, D, k_sb, k_sh, k_st, cb, st)) return rc;
+  }
+  const int64_t ws_bytes = summary_layout(B * H, T).bytes;
+  return hard(qc, kc, cb, v, dtype, B, H, T, dv, v_sb, v_sh, v_st, y, y_sb, y_sh, y_st, miss, src,
+              src_bytes, ws_bytes > 0 ? ws : nullptr, ws_bytes, st);
+}
+
 extern "C" int lema_gather(const void* v, int32_t dtype, int64_t B, int64_t H, int64_t T,
                            int64_t dv, int64_t v_sb, int64_t v_sh, int64_t v_st,
                            const void* src, int32_t src_bytes, void* y, int64_t y_sb,
