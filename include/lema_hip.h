@@ -162,6 +162,16 @@ int lema_store_exchange_ws(void* table, int64_t cap, int64_t vbytes, const void*
                            int64_t n, int64_t T, int64_t g0, int64_t* counts, int32_t* full,
                            void* workspace, int64_t workspace_bytes, void* stream);
 
+/* lema_store_exchange_ws of B * H partitions whose value rows are read in place from a
+ * [B, H, T, vbytes] view: the row of partition b * H + h, position t lies at values + b * v_sb
+ * + h * v_sh + t * v_st, BYTE strides, multiples of 8. Replaces the copy of the values ahead
+ * of the exchange (code/lema/cache.py:284-302). */
+int lema_store_exchange_view(void* table, int64_t cap, int64_t vbytes, const void* qc,
+                             const void* kc, int32_t code_bytes, const void* values, int64_t B,
+                             int64_t H, int64_t v_sb, int64_t v_sh, int64_t v_st, void* out,
+                             int64_t T, int64_t g0, int64_t* counts, int32_t* full,
+                             void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Bytes of the device scratch array behind lema_store_exchange_noalloc, per GPU. */
 #define LEMA_NOALLOC_SCRATCH_BYTES (64LL * 1024 * 1024)
 

@@ -126,7 +126,18 @@ class HashStore:
         if g0 < 0 or g0 + n // T > self.groups:
             raise ValueError(f"groups [{g0}, {g0 + n // T}) outside the store's {self.groups}")
         _lib.require_device(kc, values)
-        values = values.contiguous()
+        # a [B, H, T, d] view (a projection's values) is read in place where its strides allow and
+        # the results go to other memory
+        es = values.element_size()
+        view = (T > 1 and values.dim() == 4 and not values.is_contiguous() and values.shape[2] == T
+                and n > 0 and values.shape[0] * values.shape[1] * T == n
+                and values.shape[3] * es == self.vbytes
+                and (values.stride(3) == 1 or values.shape[3] == 1) and values.data_ptr() % 8 == 0
+                and all(s * es % 8 == 0 for s in values.stride()[:3])
+                and (out is None or out.untyped_storage().data_ptr()
+                     != values.untyped_storage().data_ptr()))
+        if not view:
+            values = values.contiguous()
         if values.numel() * values.element_size() != n * self.vbytes:
             raise ValueError(f"values hold {values.numel() * values.element_size()} bytes, "
                              f"need {n} x {self.vbytes}")
@@ -139,12 +150,20 @@ class HashStore:
         L = _lib.lib()
         ws_bytes = L.lema_store_workspace_bytes(n, T, cb)
         ws = self._workspace(ws_bytes) if ws_bytes > 0 else None
-        _lib.check(L.lema_store_exchange_ws(
-            self.table_ptr(), self.cap, self.vbytes,
-            qc.data_ptr() if qc is not None else None, kc.data_ptr(), cb, values.data_ptr(),
-            out.data_ptr() if qc is not None else None, n, T, g0,
-            self.counts_device.data_ptr(), self.full_flag.data_ptr(),
-            ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_of(kc)))
+        table, qp = self.table_ptr(), qc.data_ptr() if qc is not None else None
+        outp = out.data_ptr() if qc is not None else None
+        tail = (self.counts_device.data_ptr(), self.full_flag.data_ptr(),
+                ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_of(kc))
+        if view:
+            B, H = values.shape[:2]
+            sb, sh, st = (s * es for s in values.stride()[:3])
+            _lib.check(L.lema_store_exchange_view(
+                table, self.cap, self.vbytes, qp, kc.data_ptr(), cb, values.data_ptr(), B, H, sb,
+                sh, st, outp, T, g0, *tail))
+        else:
+            _lib.check(L.lema_store_exchange_ws(
+                table, self.cap, self.vbytes, qp, kc.data_ptr(), cb, values.data_ptr(), outp, n, T,
+                g0, *tail))
         if ws is not None and ws.numel() > self.KEEP_WORKSPACE_BYTES:
             self._ws = None       # freed once the call's kernels are done (stream-ordered)
         if check:
@@ -210,8 +229,11 @@ class LayerStore:
             qc, kc = self.codes_hook(self.layer_index, qc, kc)
         n, d_v = qc.numel(), v.shape[-1]
         got = torch.empty(v.shape, dtype=v.dtype, device=v.device)
-        self.store.exchange(qc.reshape(-1), kc.reshape(-1), v.reshape(-1, d_v),
-                            got.view(-1, d_v), n // self.partitions, self.g0, check=check)
+        T = n // self.partitions
+        if v.dim() != 4 or v.shape[0] * v.shape[1] != self.partitions or v.shape[2] != T:
+            v = v.reshape(-1, d_v)            # otherwise read in place: HashStore.exchange
+        self.store.exchange(qc.reshape(-1), kc.reshape(-1), v, got.view(-1, d_v), T, self.g0,
+                            check=check)
         return got
 
 

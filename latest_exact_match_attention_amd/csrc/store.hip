@@ -87,7 +87,9 @@ struct StoreArgs {
   const void* qc;  // null: insert only
   const void* kc;
   int32_t code_bytes;
-  const uint8_t* values;
+  const uint8_t* values;        // row of position t of partition p: value_rows(a, p) + t * v_st
+  int64_t v_sb, v_sh, v_st;     // byte strides: partition p is (p / heads, p % heads)
+  FastDiv heads;
   uint8_t* out;  // null when qc is null
   int64_t n, T, g0;
   int64_t s0;   // first position of the sub-chunk (T >= 2)
@@ -108,6 +110,15 @@ struct StoreArgs {
 __device__ __forceinline__ uint64_t code_at(const void* base, int32_t cb, int64_t i) {
   return cb == 4 ? static_cast<uint64_t>(static_cast<const uint32_t*>(base)[i])
                  : static_cast<const uint64_t*>(base)[i];
+}
+
+// The value rows of partition p, v_st bytes apart: values may be a projection viewed as
+// [B, H, T, d], read in place (the copy that made them contiguous took 37 of 162 us of a
+// 24 x 16384 call of 128-byte rows).
+__device__ __forceinline__ const uint8_t* value_rows(const StoreArgs& a, int64_t p) {
+  if (a.heads.d == 1) return a.values + p * a.v_sb;  // any number of partitions
+  const int64_t b = a.heads.div(static_cast<uint32_t>(p));
+  return a.values + b * a.v_sb + (p - b * a.heads.d) * a.v_sh;
 }
 
 __device__ __forceinline__ uint64_t* state_ptr(const StoreArgs& a, int64_t s) {
@@ -352,7 +363,7 @@ __global__ __launch_bounds__(kStepBlock) void store_step_kernel(StoreArgs a) {
   const bool has_q = a.qc != nullptr;
   const uint64_t kcode = code_at(a.kc, a.code_bytes, i);
   const uint64_t qcode = has_q ? code_at(a.qc, a.code_bytes, i) : 0;
-  const uint8_t* vrow = a.values + i * a.vbytes;
+  const uint8_t* vrow = value_rows(a, i);
   u32x4 vin = {0u, 0u, 0u, 0u};  // piece gl of the item's value row (`pre`)
   if (a.pre && gl < a.pieces) vin = *reinterpret_cast<const u32x4*>(vrow + 16 * gl);
   const int64_t khome = home_slot(kcode, tag - 2, a.cap);
@@ -432,6 +443,7 @@ __global__ __launch_bounds__(kThreads) void store_chunk_kernel(StoreArgs a) {
   const uint64_t tag = static_cast<uint64_t>(a.g0 + p) + 2;
   const int n = a.len;
   const CodeT SENT = sentinel<CodeT>();
+  const uint8_t* vrows = value_rows(a, p) + a.s0 * a.v_st;
 
   // 1. queries answered inside the sub-chunk (latest earlier key with the same code)
   if (a.qc != nullptr) {
@@ -482,7 +494,7 @@ __global__ __launch_bounds__(kThreads) void store_chunk_kernel(StoreArgs a) {
       const int j = src_in[o];
       uint8_t* dst = a.out + (first + o) * a.vbytes;
       if (j >= 0) {
-        group_copy<kGroup>(a, dst, a.values + (first + j) * a.vbytes, gl);
+        group_copy<kGroup>(a, dst, vrows + j * a.v_st, gl);
       } else {
         const uint64_t c = code_at(a.qc, a.code_bytes, first + o);
         const int64_t h = home_slot(c, tag - 2, a.cap);
@@ -503,7 +515,7 @@ __global__ __launch_bounds__(kThreads) void store_chunk_kernel(StoreArgs a) {
     const int64_t sl = group_lookup<kGroup>(a, c, tag, h, a.cap,
                                     read_window<kGroup>(a, h, a.cap, c, tag, gl, gbase), gl, gbase);
     if (sl >= 0)
-      group_copy<kGroup>(a, a.table + sl * a.stride + 16, a.values + (first + o) * a.vbytes, gl);
+      group_copy<kGroup>(a, a.table + sl * a.stride + 16, vrows + o * a.v_st, gl);
     else if (gl == 0)
       klast[o] = 2;
   }
@@ -513,7 +525,7 @@ __global__ __launch_bounds__(kThreads) void store_chunk_kernel(StoreArgs a) {
     if (klast[o] != 2) continue;
     const uint64_t c = code_at(a.kc, a.code_bytes, first + o);
     const int64_t h = home_slot(c, tag - 2, a.cap);
-    const int r = group_insert<kGroup>(a, c, tag, a.values + (first + o) * a.vbytes, h, a.cap,
+    const int r = group_insert<kGroup>(a, c, tag, vrows + o * a.v_st, h, a.cap,
                                read_window<kGroup>(a, h, a.cap, c, tag, gl, gbase), true, gl, gbase);
     if (r > 0) ++added;
     if (r < 0 && gl == 0) atomicOr(a.full, 1);
@@ -1077,7 +1089,7 @@ __global__ __launch_bounds__(256) void bulk_query_kernel(StoreArgs a, BulkWs w) 
         src = sl >= 0 ? a.table + sl * a.stride + 16 : nullptr;
       }
     }
-    if (j >= 0) src = a.values + (base + j) * a.vbytes;
+    if (j >= 0) src = value_rows(a, p) + (a.s0 + j) * a.v_st;
   }
   wave_copy_rows(a, dst, src);
 }
@@ -1092,7 +1104,7 @@ __global__ __launch_bounds__(256) void bulk_query_kernel(StoreArgs a, BulkWs w) 
 __device__ __forceinline__ int bulk_place_key(const StoreArgs& a, int64_t p, uint64_t code, int c,
                                               int32_t lp, uint8_t*& row, const uint8_t*& from) {
   const uint64_t tag = static_cast<uint64_t>(a.g0 + p) + 2;
-  from = a.values + (p * a.T + a.s0 + c * kChunk + lp) * a.vbytes;
+  from = value_rows(a, p) + (a.s0 + c * kChunk + lp) * a.v_st;
   int64_t s;
   const int r = lane_insert(a, code, tag, home_slot(code, tag - 2, a.cap), s);
   if (r < 0) atomicOr(a.full, 1);
@@ -1388,7 +1400,7 @@ bool table_in_host_memory(const void* table) {
 int store_exchange(void* table, int64_t cap, int64_t vbytes, const void* qc, const void* kc,
                    int32_t code_bytes, const void* values, void* out, int64_t n, int64_t T,
                    int64_t g0, int64_t* counts, int32_t* full, void* workspace, int64_t ws_bytes,
-                   void* stream) {
+                   void* stream, int64_t heads = 1, const int64_t* v_strides = nullptr) {
   clear_error();
   LEMA_REQUIRE(cap >= 1, "capacity must be positive, got %lld", (long long)cap);
   LEMA_REQUIRE(vbytes > 0 && vbytes % 8 == 0,
@@ -1415,6 +1427,12 @@ int store_exchange(void* table, int64_t cap, int64_t vbytes, const void* qc, con
   a.kc = kc;
   a.code_bytes = code_bytes;
   a.values = static_cast<const uint8_t*>(values);
+  // rows one behind the other unless the caller names their strides
+  a.heads = FastDiv(static_cast<uint32_t>(heads));
+  a.v_sb = v_strides != nullptr ? v_strides[0] : T * vbytes;
+  a.v_sh = v_strides != nullptr ? v_strides[1] : 0;
+  a.v_st = v_strides != nullptr ? v_strides[2] : vbytes;
+  LEMA_REQUIRE((a.v_sb | a.v_sh | a.v_st) % 8 == 0, "value strides must be multiples of 8 bytes");
   a.out = static_cast<uint8_t*>(out);
   a.n = n;
   a.T = T;
@@ -1426,6 +1444,7 @@ int store_exchange(void* table, int64_t cap, int64_t vbytes, const void* qc, con
   a.stamp_step = a.stamps != nullptr ? g_stamp_step++ : 0;
 #endif
   const bool p16 = vbytes % 16 == 0 && aligned(table, 16) && aligned(values, 16) &&
+                   (a.v_sb | a.v_sh | a.v_st) % 16 == 0 &&
                    (out == nullptr || aligned(out, 16));
   a.piece = p16 ? 16 : 8;
   a.pieces = static_cast<int32_t>(vbytes / a.piece);
@@ -1491,6 +1510,21 @@ extern "C" int lema_store_exchange_ws(void* table, int64_t cap, int64_t vbytes, 
                                       void* stream) {
   return store_exchange(table, cap, vbytes, qc, kc, code_bytes, values, out, n, T, g0, counts,
                         full, workspace, workspace_bytes, stream);
+}
+
+extern "C" int lema_store_exchange_view(void* table, int64_t cap, int64_t vbytes, const void* qc,
+                                        const void* kc, int32_t code_bytes, const void* values,
+                                        int64_t B, int64_t H, int64_t v_sb, int64_t v_sh,
+                                        int64_t v_st, void* out, int64_t T, int64_t g0,
+                                        int64_t* counts, int32_t* full, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
+  clear_error();
+  LEMA_REQUIRE(B >= 0 && H >= 1 && B < (int64_t(1) << 31) && H < (int64_t(1) << 31) &&
+                   B * H < (int64_t(1) << 31), "bad partition counts %lld x %lld", (long long)B, (long long)H);
+  LEMA_REQUIRE(v_sb >= 0 && v_sh >= 0 && v_st >= 0, "negative value strides");
+  const int64_t strides[3] = {v_sb, v_sh, v_st};
+  return store_exchange(table, cap, vbytes, qc, kc, code_bytes, values, out, B * H * T, T, g0,
+                        counts, full, workspace, workspace_bytes, stream, H, strides);
 }
 
 // ---- the exchange without a workspace argument and without allocation ----
