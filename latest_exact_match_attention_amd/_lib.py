@@ -128,8 +128,9 @@ def check(status: int) -> None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    """The raw hipStream_t of the current torch stream on t's device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw hipStream_t of the current torch stream on t's device (0.1 us; a Stream object
+    of current_stream() takes 1.8)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 # ---- host memory the GPU works on in place (a store table in host RAM) ----

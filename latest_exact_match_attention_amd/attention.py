@@ -214,9 +214,9 @@ def _hard_z(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     y = torch.empty_like(v)
     if y.stride(3) != 1 and dv > 1:
         y = torch.empty(v.shape, dtype=v.dtype, device=v.device)
-    src = torch.empty((B, H, T), dtype=torch.int32, device=v.device) if want_src else None
+    src = v.new_empty((B, H, T), dtype=torch.int32) if want_src else None
     n = L.lema_hard_z_workspace_bytes(B * H, T, 4 if D <= 32 else 8)
-    ws = torch.empty(n, dtype=torch.uint8, device=v.device)
+    ws = v.new_empty(n, dtype=torch.uint8)
     qs, ks, vs, ys = q.stride(), k.stride(), v.stride(), y.stride()
     _lib.check(L.lema_hard_z(
         q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[q.dtype], D, qs[0], qs[1], qs[2], ks[0], ks[1],

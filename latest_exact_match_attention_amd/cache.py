@@ -228,7 +228,7 @@ class LayerStore:
         if self.codes_hook is not None:       # on the device, inside a captured step
             qc, kc = self.codes_hook(self.layer_index, qc, kc)
         n, d_v = qc.numel(), v.shape[-1]
-        got = torch.empty(v.shape, dtype=v.dtype, device=v.device)
+        got = v.new_empty(v.shape)
         T = n // self.partitions
         if v.dim() != 4 or v.shape[0] * v.shape[1] != self.partitions or v.shape[2] != T:
             v = v.reshape(-1, d_v)            # otherwise read in place: HashStore.exchange

@@ -50,7 +50,10 @@ __all__ = ["ModelConfig", "SwiGLU", "Attention", "Block", "Transformer", "lm_los
 # run as one HIP kernel each (liblema_hip.so); other dtypes and devices use the torch ops.
 
 def _fused(*ts: torch.Tensor) -> bool:
-    return all(t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous() for t in ts)
+    for t in ts:
+        if not (t.is_cuda and t.dtype is torch.bfloat16 and t.is_contiguous()):
+            return False
+    return True
 
 
 def rms_norm(x: torch.Tensor, norm: nn.RMSNorm, d: torch.Tensor | None = None):
@@ -135,7 +138,7 @@ def linear(x: torch.Tensor, lin: nn.Linear) -> torch.Tensor:
         return lin(x)
     K, N = x.shape[-1], lin.weight.shape[0]
     M = x.numel() // K
-    y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+    y = x.new_empty(x.shape[:-1] + (N,))
     _lib.check(_lib.lib().lema_skinny_gemm_bf16(
         x.data_ptr(), K, lin.weight.data_ptr(), K, y.data_ptr(), N, M, N, K, _lib.stream_of(x)))
     return y
@@ -183,9 +186,9 @@ def project_qkv(x: torch.Tensor, at, code_dtype: torch.dtype, norm: nn.RMSNorm |
                 and K <= 2048
                 and M * (K + 8) * 2 + 8 * (16 if M <= 16 else 32) * (16 * ct + 1) * 4 <= 160 * 1024):
             return None
-    qc = torch.empty((B, Nqk // c.d_qk, T), dtype=code_dtype, device=x.device)
+    qc = x.new_empty((B, Nqk // c.d_qk, T), dtype=code_dtype)
     kc = torch.empty_like(qc)
-    v = torch.empty((B, T, Nv), dtype=x.dtype, device=x.device)
+    v = x.new_empty((B, T, Nv))
     if norm is not None:
         eps = norm.eps if norm.eps is not None else torch.finfo(x.dtype).eps
         _lib.check(_lib.lib().lema_skinny_norm_qkv_bf16(
@@ -310,7 +313,7 @@ class SwiGLU(nn.Module):
         if _skinny(x, g) and g.shape == u.shape and u.data_ptr() % 16 == 0 and u.is_contiguous():
             K, N = x.shape[-1], g.shape[0]
             M = x.numel() // K
-            a = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+            a = x.new_empty(x.shape[:-1] + (N,))
             _lib.check(_lib.lib().lema_skinny_swiglu_bf16(
                 x.data_ptr(), K, g.data_ptr(), u.data_ptr(), K, M, N, K, a.data_ptr(),
                 _lib.stream_of(x)))
@@ -351,7 +354,7 @@ class SwiGLU(nn.Module):
                 and _fused(dn) and dn.data_ptr() % 16 == 0 and N % 32 == 0):
             return None
         xo = torch.empty_like(x)
-        a = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+        a = x.new_empty(x.shape[:-1] + (N,))
         eps = norm.eps if norm.eps is not None else torch.finfo(x.dtype).eps
         _lib.check(_lib.lib().lema_skinny_norm_swiglu_bf16(
             x.data_ptr(), d.data_ptr(), norm.weight.data_ptr(), float(eps), xo.data_ptr(),
