@@ -125,20 +125,33 @@ __device__ __forceinline__ uint64_t* state_ptr(const StoreArgs& a, int64_t s) {
   return reinterpret_cast<uint64_t*>(a.table + s * a.stride) + 1;
 }
 
-// Copy one value row with the group's lanes (src null: write zeros).
+// Copy one value row with the group's lanes (src null: write zeros). A lane's pieces are all
+// loaded (up to 4 at a time) before the first is stored: with a load and a store by turns, each
+// of a lane's four pieces of a 128-byte row waited for the one before (chunked calls of 1024 x
+// 1024 positions, new keys: 447 -> 395 us, overwrites 398 -> 305 us; 96 x 200: 31.3 -> 29.2 and
+// 20.2 -> 18.4 us).
+template <int G, typename Piece>
+__device__ __forceinline__ void group_copy_pieces(uint8_t* dst, const uint8_t* src, int pieces, int gl) {
+  constexpr int kFlight = 4;
+  for (int k0 = gl; k0 < pieces; k0 += kFlight * G) {
+    Piece v[kFlight];
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) {
+      v[u] = Piece(0u);
+      if (src != nullptr && k0 + u * G < pieces) v[u] = reinterpret_cast<const Piece*>(src)[k0 + u * G];
+    }
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u)
+      if (k0 + u * G < pieces) reinterpret_cast<Piece*>(dst)[k0 + u * G] = v[u];
+  }
+}
 template <int G>
 __device__ __forceinline__ void group_copy(const StoreArgs& a, uint8_t* dst, const uint8_t* src,
                                            int gl) {
-  const int pieces = static_cast<int>(a.vbytes / a.piece);
-  for (int k = gl; k < pieces; k += G) {
-    if (a.piece == 16) {
-      const u32x4 v = src ? *reinterpret_cast<const u32x4*>(src + 16 * k) : u32x4{0u, 0u, 0u, 0u};
-      *reinterpret_cast<u32x4*>(dst + 16 * k) = v;
-    } else {
-      const u32x2 v = src ? *reinterpret_cast<const u32x2*>(src + 8 * k) : u32x2{0u, 0u};
-      *reinterpret_cast<u32x2*>(dst + 8 * k) = v;
-    }
-  }
+  if (a.piece == 16)
+    group_copy_pieces<G, u32x4>(dst, src, a.pieces, gl);
+  else
+    group_copy_pieces<G, u32x2>(dst, src, a.pieces, gl);
 }
 
 // Copy the value rows the lanes of a wave name (lane L: dst_L non-null; src_L null writes
