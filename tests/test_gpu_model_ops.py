@@ -132,3 +132,20 @@ def test_device_copy(dev):
         assert not dst[4 * n16:].any(), n16           # nothing written past the end
     with pytest.raises(ValueError):
         _lib.check(_lib.lib().lema_device_copy(src.data_ptr(), dst.data_ptr(), 24, st))
+
+
+@pytest.mark.parametrize("V", [8, 8192, 65536 + 8, 70000])
+def test_argmax_signed_zeros_and_groups(dev, V):
+    """-0 and +0 tie (the first wins), negative NaNs win too, and the maximum may lie in any
+    group of pieces, the last piece of the row included."""
+    from latest_exact_match_attention_amd.model import argmax_into
+    x = torch.full((6, 1, V), -3.0, device=dev, dtype=torch.bfloat16)
+    x[0, 0, V // 2], x[0, 0, V - 1] = -0.0, 0.0
+    x[1, 0, 3], x[1, 0, V - 2] = 0.0, -0.0
+    x[2, 0, V - 1] = -2.0
+    x[3, 0, V - 4] = -float("nan")
+    x[4, 0, V - 8:] = float("inf")
+    x[5] = -float("inf")
+    out = torch.full((6, 1), -9, dtype=torch.long, device=dev)
+    argmax_into(x, out)
+    assert out.view(-1).tolist() == [V // 2, 3, V - 1, V - 4, V - 8, 0]
