@@ -862,6 +862,7 @@ def bench_long(a):
                   "counts_identical_after_checked_calls": counts_same}
     if full_par is not None:
         parity = dict(parity or {}, reference_store_calls=n_par, all_calls=full_par)
+    if cpu_s:
         cpu = {"value": H * L * n_par / sum(cpu_s), "unit": "queries/s", "cores": threads,
                "kind": "reference", "cpu_model": cpu_model(),
                "sample": f"the first {n_par} call(s) of 64 x 2^20 positions through "
