@@ -115,6 +115,15 @@ __device__ __forceinline__ bool bf16_nonneg(float z) {
   return bf16_bits_to_f32(f32_to_bf16_bits(z)) >= 0.0f;
 }
 
+// Exchanges the values of lanes 8 apart in each row of 16 lanes.
+__device__ __forceinline__ u32x4 swap_halves(u32x4 v) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    r[i] = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v[i]), 0x128, 0xf, 0xf, true));
+  return r;
+}
+
 // A block owns `cols` columns: 16 * CT, or 8 for a narrow plain segment (swiglu: 16 columns
 // of the gate and the same 16 of up). kNorm: 0 = x as it is, 1 = norm(x), 2 = norm(x + nd).
 //
@@ -127,14 +136,18 @@ __device__ __forceinline__ bool bf16_nonneg(float z) {
 // of its share (6 steps for K of up to 1536, 8 up to 2048), and the weights' loads are issued
 // before the pre-norm's arithmetic and arrive meanwhile.
 //
-// kHalf: a narrow block (8 columns) of at most 8 rows fills the matrix tile's idle quarters with
-// a second K-step: columns and rows 8..15 are the same columns and rows one step on, and the
-// two diagonal quarters of the result are added in the reduction. Half the load instructions
-// (the lanes past the block's columns would repeat others' loads at the same cost).
+// kHalf: a narrow block (8 columns) of at most 8 rows loads a second K-step into the matrix
+// tile's idle quarters: columns and rows 8..15 are the same columns and rows one step on. Half
+// the load instructions (the lanes past the block's columns would repeat others' loads at the
+// same cost). The second step is multiplied after the first, both operands' halves exchanged by
+// data-parallel moves, so a column adds its products in the order of a full tile and its bits
+// don't depend on how many rows the call has (the two steps summed apart and added at the
+// end differed from that in the last places, and a decoder's logits with them).
 //
 // Measured, launches in a graph over weights from HBM, before and now: M = 1, K = 1536,
-// N = 1536 4.60 and 3.57 us, N = 4096 5.49 and 4.71, N = 8192 8.26 and 6.92; K = 4096, N = 1536
-// 6.96 and 5.03; M = 16, N = 8192 10.9 and 8.9.
+// N = 1536 4.60 and 3.71 us, N = 4096 5.49 and 4.71, N = 8192 8.26 and 6.92; K = 4096, N = 1536
+// 6.96 and 5.16; M = 16, N = 8192 10.9 and 8.9. (Half-filled tiles whose steps were summed apart:
+// 3.64 and 5.14.)
 template <int MT, int CT, int kNorm, int U, bool kHalf>
 __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 4 : 2) void skinny_kernel(SkDevice a) {
   constexpr int kSteps = U == 6 ? kSkShortK / 512 : kSkNormSteps;  // the norm's
@@ -158,12 +171,13 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
   const int64_t ldx = static_cast<int64_t>(a.ldx8) * 8, ldw = static_cast<int64_t>(a.ldw8) * 8;
   const int n0 = bid * cols;
-  const int ksteps = a.K / (kHalf ? 64 : 32);
-  constexpr int kStep = kHalf ? 64 : 32;
+  const int ksteps = a.K / 32;
   const int per = (ksteps + kSkWaves - 1) / kSkWaves;
   const int s0 = wave * per;
   const int s1 = s0 + per < ksteps ? s0 + per : ksteps;
-  const int last = s1 > 0 ? s1 - 1 : 0;  // the step that loads past the share repeat
+  // the step (kHalf: the two steps) that loads past the share repeat
+  const int last = s1 > (kHalf ? 2 : 1) ? s1 - (kHalf ? 2 : 1) : 0;
+  constexpr int kGroup = kHalf ? 2 * U : U;  // K-steps of a group
   const int r16 = l & 15, kg = (l >> 4) * 8;
 
   const uint16_t* wp[CT];
@@ -179,10 +193,15 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
   // took them apart into elements and reused half of one fragment's registers for an address
   typedef u32x4 WFrag[U][CT];
   typedef u32x4 XFrag[U][MT];
+  // the step that load u of the group at s begins with, in bounds
+  auto step_at = [&](int s, int u) __attribute__((always_inline)) {
+    if constexpr (kHalf) return s + 2 * u < last ? s + 2 * u : last;
+    return s + u < s1 ? s + u : last;
+  };
   auto load_w = [&](WFrag& f, int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int at = (s + u < s1 ? s + u : last) * kStep;
+      const int at = step_at(s, u) * 32;
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) f[u][ct] = *reinterpret_cast<const u32x4*>(wp[ct] + at);
     }
@@ -246,10 +265,14 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
   auto load_x = [&](XFrag& f, int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int at = (s + u < s1 ? s + u : last) * kStep;
+      const int at = step_at(s, u) * 32;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) f[u][mt] = *reinterpret_cast<const u32x4*>(xp[mt] + at);
     }
+  };
+  auto product = [&](int mt, int ct, u32x4 x, u32x4 w) __attribute__((always_inline)) {
+    acc[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, w),
+                                                          acc[mt][ct], 0, 0, 0);
   };
   // `end`: the share may end inside the group. Steps past it are left out, with x from memory; with
   // x from LDS they multiply zeros (both factors, so that a stray infinity adds nothing): a
@@ -267,13 +290,21 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (kNorm == 0 && end && s + u >= s1) break;  // the same in every lane
+      if constexpr (kHalf) {
+        const int at = s + 2 * u;  // the same in every lane, as s1 and last
+        // an odd share's last step was loaded as the second of its pair
+        if (!end || (at < s1 && at <= last)) product(0, 0, x[u][0], w[u][0]);
+        // the swaps take copies as far as the compiler knows: with both products reading the same
+        // fragments it reused two of a fragment's registers before the first one had read them
+        asm("" : "+v"(x[u][0]), "+v"(w[u][0]));
+        if (!end || (at < s1 && (at + 1 < s1 || at > last))) product(0, 0, swap_halves(x[u][0]), swap_halves(w[u][0]));
+      } else {
+        if (kNorm == 0 && end && s + u >= s1) break;  // the same in every lane
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-          acc[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, x[u][mt]), __builtin_bit_cast(bf16x8, w[u][ct]), acc[mt][ct], 0, 0, 0);
+          for (int ct = 0; ct < CT; ++ct) product(mt, ct, x[u][mt], w[u][ct]);
+      }
     }
   };
   XFrag xa;
@@ -285,22 +316,22 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
     XFrag xb;
     int s = s0;
     for (;;) {  // two groups a trip, so that neither is copied
-      if (s + U >= s1) {
+      if (s + kGroup >= s1) {
         products(wa, xa, s, true);
         break;
       }
-      load_w(wb, s + U);
-      load_x(xb, s + U);
+      load_w(wb, s + kGroup);
+      load_x(xb, s + kGroup);
       products(wa, xa, s, false);
-      s += U;
-      if (s + U >= s1) {
+      s += kGroup;
+      if (s + kGroup >= s1) {
         products(wb, xb, s, true);
         break;
       }
-      load_w(wa, s + U);
-      load_x(xa, s + U);
+      load_w(wa, s + kGroup);
+      load_x(xa, s + kGroup);
       products(wb, xb, s, false);
-      s += U;
+      s += kGroup;
     }
   }
 #pragma unroll
@@ -321,10 +352,7 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
     if (e < kRows * kCols) {
       const int row = e / kCols, col = e - (e / kCols) * kCols;
 #pragma unroll
-      for (int wv = 0; wv < kSkWaves; ++wv) {
-        sums[i] += part[wv][row][col];
-        if constexpr (kHalf) sums[i] += part[wv][(row + 8) & 15][(col + 8) & 15];
-      }
+      for (int wv = 0; wv < kSkWaves; ++wv) sums[i] += part[wv][row][col];
     }
   }
   if (mode == kSkPlain) {
@@ -456,9 +484,9 @@ int launch_skinny(SkinnyArgs& a, hipStream_t st) {
   } else if constexpr (CT == 1) {
     // K-steps per group: the larger one unless it divides a wavefront's share worse
     const int per = (a.K / 32 + kSkWaves - 1) / kSkWaves;
-    const int half = (a.K / 64 + kSkWaves - 1) / kSkWaves;
+    const int half = (per + 1) / 2;  // pairs of steps
     auto waste = [](int share, int u) { return (share + u - 1) / u * u - share; };
-    if (narrow && a.M <= 8 && a.K % 64 == 0)
+    if (narrow && a.M <= 8 && a.K >= 64)
       kernel = waste(half, 4) <= waste(half, 3) ? skinny_kernel<1, 1, 0, 4, true> : skinny_kernel<1, 1, 0, 3, true>;
     else if (waste(per, 6) <= waste(per, 4))
       kernel = a.M <= 16 ? skinny_kernel<1, 1, 0, 6, false> : skinny_kernel<2, 1, 0, 6, false>;

@@ -40,6 +40,20 @@ def test_shares(dev, M, N, K):
     assert float(((_product(x, w).double() - ref).abs() - bound).max()) <= 0.0
 
 
+@pytest.mark.parametrize("K", [32, 64, 96, 256, 288, 512, 768, 1536, 1568, 2816, 4096, 6144])
+@pytest.mark.parametrize("N", [5, 24, 1536, 2048])
+def test_bits_do_not_depend_on_the_other_rows(dev, N, K):
+    """A row's products are added in one order, whatever the number of rows: up to 8 of them in a
+    half-filled tile, 9 and more in a full one, 17 and more in two."""
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    x = torch.randn((17, K), device=dev, generator=g).to(torch.bfloat16)
+    w = (torch.randn((N, K), device=dev, generator=g) * K ** -0.5).to(torch.bfloat16)
+    want = _product(x[:9], w)
+    for M in (1, 3, 8):
+        assert torch.equal(_product(x[:M].contiguous(), w), want[:M]), M
+    assert torch.equal(_product(x, w)[:9], want)
+
+
 def test_an_infinity_stays_in_its_products(dev):
     """An infinity in the last column of x or a weight touches its own row or column alone."""
     for K in (1536, 1792, 2048):
