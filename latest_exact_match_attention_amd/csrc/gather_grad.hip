@@ -50,18 +50,27 @@ struct GradArgs {
   int64_t row_bytes;
   int32_t pieces;      // pieces per value row
   int32_t R, nch;      // source rows per workgroup, workgroups per row
-  int32_t group;       // 8 consecutive rows per XCD, one part of all 8 in a row (gg_item)
+  int32_t order;       // of the workgroups (gg_item)
   FastDiv pdiv;        // division by `pieces`
 };
 
-// (row, part) of workgroup v, of `parts` per row. Workgroup v runs on XCD v % 8. When the rows
-// come in whole groups of 64, rows 8g..8g+7 belong to XCD g % 8, which takes a part of all 8
-// back to back: where gy interleaves the rows (a projection view), their pieces of each line
-// are then read through one L2. Otherwise row r runs on XCD r % 8. First parts first: they have
-// the most indices to scan.
-__device__ __forceinline__ void gg_item(bool group, int parts, int v, int64_t& row, int& part) {
+// (row, part) of workgroup v, of `parts` per row. Workgroup v runs on XCD v % 8.
+//   kGgGroups  N a multiple of 64: rows 8g..8g+7 belong to XCD g % 8, which takes a part of all 8
+//              back to back: where gy interleaves the rows (a projection view), their pieces of
+//              each line are then read through one L2
+//   kGgRowXcd  N a multiple of 8: row r runs on XCD r % 8, whose L2 keeps its indices
+//   kGgSpread  any other N: a row's parts go round the XCDs. Bound to an XCD each, the rows left
+//              8 - N of the XCDs idle for N < 8 (N = 1: all but 32 CUs)
+// First parts first: they have the most indices to scan.
+constexpr int kGgSpread = 0, kGgRowXcd = 1, kGgGroups = 2;
+__device__ __forceinline__ void gg_item(int order, int64_t N, int parts, int v, int64_t& row, int& part) {
+  if (order == kGgSpread) {
+    part = v / static_cast<int>(N);
+    row = v - part * static_cast<int>(N);
+    return;
+  }
   const int xcd = v % kNumXcd, k = v / kNumXcd;
-  if (group) {
+  if (order == kGgGroups) {
     const int per = kNumXcd * parts;
     part = (k % per) / kNumXcd;
     row = (static_cast<int64_t>(k / per) * kNumXcd + xcd) * kNumXcd + (k % per) % kNumXcd;
@@ -178,8 +187,7 @@ __global__ __launch_bounds__(kGgThreads) void gather_grad_kernel(GradArgs a) {
   const int t = threadIdx.x, lane = t & 63;
   int64_t row;
   int part_no;
-  gg_item(a.group != 0, a.nch, blockIdx.x, row, part_no);
-  if (row >= a.N) return;
+  gg_item(a.order, a.N, a.nch, blockIdx.x, row, part_no);
   const int64_t j0 = static_cast<int64_t>(part_no) * a.R;
   const int rows = static_cast<int>(a.T - j0 < a.R ? a.T - j0 : a.R);
   const int32_t* src = a.src + row * a.T;
@@ -368,8 +376,7 @@ __global__ __launch_bounds__(kGgThreads) void gather_grad_miss_kernel(GradArgs a
   const int t = threadIdx.x, lane = t & 63;
   int64_t row;
   int part_no;
-  gg_item(a.group != 0, nch, blockIdx.x, row, part_no);
-  if (row >= a.N) return;
+  gg_item(a.order, a.N, nch, blockIdx.x, row, part_no);
   if (t == 0) count = 0;
   __syncthreads();
   const int64_t i = static_cast<int64_t>(part_no) * kMissPositions + t;
@@ -412,19 +419,19 @@ __global__ __launch_bounds__(kGgThreads) void gather_grad_miss_kernel(GradArgs a
 
 template <int DTYPE, int VEC>
 int launch_grad(GradArgs& a, hipStream_t st) {
-  const int64_t rows8 = (a.N + kNumXcd - 1) / kNumXcd * kNumXcd;
   // Fewer source rows per workgroup while the launch has under 4 workgroups per CU
   a.R = kGgRows;
-  while (a.R > 64 && rows8 * ((a.T + a.R - 1) / a.R) < 1024) a.R /= 2;
+  while (a.R > 64 && a.N * ((a.T + a.R - 1) / a.R) < 1024) a.R /= 2;
   const int64_t nch = (a.T + a.R - 1) / a.R;
   const int64_t mch = (a.T + kMissPositions - 1) / kMissPositions;
-  LEMA_REQUIRE(rows8 * mch < (int64_t(1) << 31), "too many rows x positions");
+  LEMA_REQUIRE(a.N < (int64_t(1) << 31) && a.N * mch < (int64_t(1) << 31) && a.N * nch < (int64_t(1) << 31),
+               "too many rows x positions");
   a.nch = static_cast<int32_t>(nch);
-  a.group = a.N % 64 == 0;
-  gather_grad_kernel<DTYPE, VEC><<<dim3(rows8 * nch), dim3(kGgThreads), 0, st>>>(a);
+  a.order = a.N % 64 == 0 ? kGgGroups : a.N % kNumXcd == 0 ? kGgRowXcd : kGgSpread;
+  gather_grad_kernel<DTYPE, VEC><<<dim3(a.N * nch), dim3(kGgThreads), 0, st>>>(a);
   if (int rc = launch_status("gather_grad_kernel")) return rc;
   gather_grad_miss_kernel<DTYPE, VEC>
-      <<<dim3(rows8 * mch), dim3(kGgThreads), 0, st>>>(a, static_cast<int32_t>(mch));
+      <<<dim3(a.N * mch), dim3(kGgThreads), 0, st>>>(a, static_cast<int32_t>(mch));
   return launch_status("gather_grad_miss_kernel");
 }
 

@@ -59,6 +59,9 @@ def _view(x, form):
     ("many", 2, 64, 3000, 24, "projection"), ("first", 1, 8, 5000, 16, "plain"),
     ("first", 1, 1, 9001, 520, "projection"), ("spread", 2, 3, 20000, 8, "plain"),
     ("spread", 1, 128, 9000, 4, "projection"), ("few", 1, 2, 700, 1100, "columns"),
+    # rows that don't fill the XCDs: their parts go round them
+    ("few", 1, 1, 40001, 8, "plain"), ("many", 1, 7, 5003, 24, "projection"), ("spread", 3, 3, 2600, 16, "plain"),
+    ("few", 1, 12, 1500, 24, "projection"), ("first", 1, 8, 2050, 8, "offset"),
 ])
 def test_gradient_is_the_sum(dev, dtype, kind, B, H, T, dv, form):
     g = torch.Generator().manual_seed(T + dv)
