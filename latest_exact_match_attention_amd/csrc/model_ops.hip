@@ -182,9 +182,14 @@ extern "C" int lema_rmsnorm_bf16(const void* x, const void* d, const void* w, fl
                "pointers must be 16-byte aligned");
   const int64_t grid = (rows + 3) / 4;
   LEMA_REQUIRE(grid < (int64_t(1) << 31), "too many rows");
-  // rows of up to 1536 or 2048 (the models' widths) hold 3 or 4 steps in registers, longer
-  // ones 8
-  auto kernel = D <= 1536 ? rmsnorm_kernel<3> : D <= 2048 ? rmsnorm_kernel<4> : rmsnorm_kernel<kNormMaxSteps>;
+  // As many steps of 512 elements as the row has, up to 4; longer rows hold 8. Every step of the
+  // kernel loads, so one with 3 steps took 33.8 us for 65,536 rows of 256 with an addend (30.0 with a
+  // kernel that skips them).
+  auto kernel = D <= 512    ? rmsnorm_kernel<1>
+                : D <= 1024 ? rmsnorm_kernel<2>
+                : D <= 1536 ? rmsnorm_kernel<3>
+                : D <= 2048 ? rmsnorm_kernel<4>
+                            : rmsnorm_kernel<kNormMaxSteps>;
   kernel<<<dim3(grid), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(d),
       static_cast<const uint16_t*>(w), eps, rows, static_cast<int>(D),
@@ -201,27 +206,29 @@ __device__ __forceinline__ uint32_t argmax_key(uint32_t u) {
 
 // One workgroup (1024 threads) per row of V bf16 values (V % 8 == 0, rows 16-byte aligned):
 // out[row * out_stride] = the row's argmax (code/lema/decode.py:71-93, the greedy pick). Bound by
-// one CU's reads: a thread has 8 pieces in flight and keeps (key, earlier first) in one 32-bit
+// one CU's reads: a thread has F pieces in flight and keeps (key, earlier first) in one 32-bit
 // word per group of them, (key, index) in 64 bits across groups. With a piece loaded and
-// compared at a time a row of 50,304 took 12.3 us, now 6.4.
-constexpr int kArgmaxFlight = 8;
+// compared at a time a row of 50,304 took 12.3 us, with 8 in flight 6.4. F is what the row has for
+// a thread, 1, 2, 4 or 8: a group always loads and compares F (4096 rows of 8192 took 92.8 us
+// with 8, 50.7 with a piece at a time).
 constexpr uint64_t kArgmaxIndex = (uint64_t(1) << 48) - 1;
+template <int F>
 __global__ __launch_bounds__(1024) void argmax_kernel(const uint16_t* x, int64_t V, int64_t ld,
                                                       int64_t* out, int64_t out_stride) {
   __shared__ uint64_t best_of[16];
   const int64_t row = blockIdx.x;
   const uint16_t* r = x + row * ld;
   uint64_t best = 0;  // key << 48 | (2^48 - 1 - index); every element's is above 0
-  for (int64_t e0 = static_cast<int64_t>(threadIdx.x) * 8; e0 < V; e0 += kArgmaxFlight * 1024 * 8) {
-    u32x4 v[kArgmaxFlight];
+  for (int64_t e0 = static_cast<int64_t>(threadIdx.x) * 8; e0 < V; e0 += F * 1024 * 8) {
+    u32x4 v[F];
 #pragma unroll
-    for (int u = 0; u < kArgmaxFlight; ++u) {
+    for (int u = 0; u < F; ++u) {
       const int64_t e = e0 + u * 1024 * 8;
       v[u] = *reinterpret_cast<const u32x4*>(r + (e < V ? e : e0));  // past the row: the first again
     }
     uint32_t top = 0;  // key << 16 | (0xFFFF - place among the thread's 64)
 #pragma unroll
-    for (int u = 0; u < kArgmaxFlight; ++u) {
+    for (int u = 0; u < F; ++u) {
       const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -282,7 +289,11 @@ extern "C" int lema_argmax_bf16(const void* x, int64_t rows, int64_t V, int64_t 
   if (rows == 0) return LEMA_OK;
   LEMA_REQUIRE(x && out && aligned(x, 16) && aligned(out, 8) && out_stride >= 1, "bad pointer");
   LEMA_REQUIRE(rows < (int64_t(1) << 31), "too many rows");
-  argmax_kernel<<<dim3(rows), dim3(1024), 0, static_cast<hipStream_t>(stream)>>>(
+  const auto kernel = V <= 8192    ? argmax_kernel<1>
+                      : V <= 16384 ? argmax_kernel<2>
+                      : V <= 32768 ? argmax_kernel<4>
+                                   : argmax_kernel<8>;
+  kernel<<<dim3(rows), dim3(1024), 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(x), V, ld, out, out_stride);
   return launch_status("argmax_kernel");
 }

@@ -39,8 +39,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSkThreads = 512;
 constexpr int kSkWaves = kSkThreads / 64;
-constexpr int kSkShortK = 1536;  // rows of up to this (kShort) or kSkNormSteps * 512 elements
-constexpr int kSkNormSteps = 4;  // a fused pre-norm's rows: up to 4 * 512 elements in registers
+constexpr int kSkStepK = 32 * kSkWaves;  // row elements that give every wavefront one K-step
+constexpr int kSkNormMaxK = 8 * kSkStepK;  // longest rows of a fused pre-norm, held in registers
 
 // One weight segment of a launch: its blocks cover N output columns of x . w^T with one
 // epilogue. A launch holds up to three segments sharing x (the q, k and v projections of a
@@ -131,10 +131,14 @@ __device__ __forceinline__ u32x4 swap_halves(u32x4 v) {
 // lanes without a column or row of their own, and steps past a wavefront's share, read
 // in-bounds elements whose products nothing uses. With a load per branch the compiler waited
 // for every load of a group of 4 steps before its products and issued the next group after
-// them. U is the K-steps of a group; the next group's loads are issued before the current one's
-// products, so a wavefront has one to two groups in flight. With a pre-norm one group is all
-// of its share (6 steps for K of up to 1536, 8 up to 2048), and the weights' loads are issued
-// before the pre-norm's arithmetic and arrive meanwhile.
+// them. U is the K-steps of a group (kHalf: pairs of steps). A wavefront whose share is more than
+// a group (kMore) issues the next group's loads before the current one's products, so it has
+// one to two groups in flight. With a pre-norm one group is all of its share (3, 4, 6 or 8 steps
+// for K of up to 768, 1024, 1536 or 2048), and the weights' loads are issued before the
+// pre-norm's arithmetic and arrive meanwhile. Steps past the share cost a load each, and a second
+// group's registers keep other workgroups off the CU: K = 768, N = 50304 (3 steps) took
+// 22.6 us at M = 1 and 42.6 at M = 17 with groups of 4 and room for two, NEW1 and NEW17 now
+// (16.4 and 27.4 with every load conditional).
 //
 // kHalf: a narrow block (8 columns) of at most 8 rows loads a second K-step into the matrix
 // tile's idle quarters: columns and rows 8..15 are the same columns and rows one step on. Half
@@ -148,10 +152,10 @@ __device__ __forceinline__ u32x4 swap_halves(u32x4 v) {
 // N = 1536 4.60 and 3.71 us, N = 4096 5.49 and 4.71, N = 8192 8.26 and 6.92; K = 4096, N = 1536
 // 6.96 and 5.16; M = 16, N = 8192 10.9 and 8.9. (Half-filled tiles whose steps were summed apart:
 // 3.64 and 5.14.)
-template <int MT, int CT, int kNorm, int U, bool kHalf>
+template <int MT, int CT, int kNorm, int U, bool kHalf, bool kMore>
 __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 4 : 2) void skinny_kernel(SkDevice a) {
-  constexpr int kSteps = U == 6 ? kSkShortK / 512 : kSkNormSteps;  // the norm's
-  static_assert(kNorm == 0 || 512 * kSteps <= 32 * kSkWaves * U, "one group of loads");
+  constexpr int kSteps = (kSkStepK * U + 511) / 512;  // the norm's, of 512 elements
+  static_assert(kNorm == 0 || !kMore, "one group of loads");
   static_assert(!kHalf || (MT == 1 && CT == 1 && kNorm == 0), "a half-filled tile");
   __shared__ float part[kSkWaves][MT * 16][CT * 16 + 1];
   extern __shared__ __align__(16) uint16_t xs[];  // kNorm: the normalised rows, stride K + 8
@@ -309,7 +313,9 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
   };
   XFrag xa;
   load_x(xa, s0);
-  if constexpr (kNorm != 0) {
+  if constexpr (!kMore) {
+    // no load moves past this into the branch of the product that uses it
+    if constexpr (kNorm == 0) asm volatile("" ::: "memory");
     products(wa, xa, s0, true);
   } else {
     WFrag wb;
@@ -474,26 +480,48 @@ int launch_skinny(SkinnyArgs& a, hipStream_t st) {
   const dim3 grid(blocks), block(kSkThreads);
   const size_t lds = a.nw != nullptr ? static_cast<size_t>(a.M) * (a.K + 8) * sizeof(uint16_t) : 0;
   void (*kernel)(SkDevice) = nullptr;
+  const int per = (a.K / 32 + kSkWaves - 1) / kSkWaves;  // K-steps of a wavefront
   if (a.nw != nullptr) {  // the normalised rows in LDS (checked to fit by the entry point)
+    auto pick_u = [&](auto mt, auto norm) {
+      constexpr int MT = decltype(mt)::value, kNorm = decltype(norm)::value;
+      if constexpr (CT <= 2) {  // whole-head codes of other widths (CT 3) are rare: two sizes
+        if (per <= 3) return skinny_kernel<MT, CT, kNorm, 3, false, false>;
+        if (per <= 4) return skinny_kernel<MT, CT, kNorm, 4, false, false>;
+      }
+      return per <= 6 ? skinny_kernel<MT, CT, kNorm, 6, false, false> : skinny_kernel<MT, CT, kNorm, 8, false, false>;
+    };
     auto pick = [&](auto mt) {
-      constexpr int MT = decltype(mt)::value;
-      return a.nd != nullptr ? (a.K <= kSkShortK ? skinny_kernel<MT, CT, 2, 6, false> : skinny_kernel<MT, CT, 2, 8, false>)
-                             : (a.K <= kSkShortK ? skinny_kernel<MT, CT, 1, 6, false> : skinny_kernel<MT, CT, 1, 8, false>);
+      return a.nd != nullptr ? pick_u(mt, std::integral_constant<int, 2>{}) : pick_u(mt, std::integral_constant<int, 1>{});
     };
     kernel = a.M <= 16 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
   } else if constexpr (CT == 1) {
-    // K-steps per group: the larger one unless it divides a wavefront's share worse
-    const int per = (a.K / 32 + kSkWaves - 1) / kSkWaves;
+    // steps past a share of `n` in groups of u; the larger group unless it divides the share worse
+    auto waste = [](int n, int u) { return (n + u - 1) / u * u - n; };
     const int half = (per + 1) / 2;  // pairs of steps
-    auto waste = [](int share, int u) { return (share + u - 1) / u * u - share; };
+    auto pick = [&](auto mt) {
+      constexpr int MT = decltype(mt)::value;
+      if (per <= 3) return skinny_kernel<MT, 1, 0, 3, false, false>;
+      if (per <= 4) return skinny_kernel<MT, 1, 0, 4, false, false>;
+      if (per <= 6) return skinny_kernel<MT, 1, 0, 6, false, false>;
+      return waste(per, 6) <= waste(per, 4) ? skinny_kernel<MT, 1, 0, 6, false, true> : skinny_kernel<MT, 1, 0, 4, false, true>;
+    };
     if (narrow && a.M <= 8 && a.K >= 64)
-      kernel = waste(half, 4) <= waste(half, 3) ? skinny_kernel<1, 1, 0, 4, true> : skinny_kernel<1, 1, 0, 3, true>;
-    else if (waste(per, 6) <= waste(per, 4))
-      kernel = a.M <= 16 ? skinny_kernel<1, 1, 0, 6, false> : skinny_kernel<2, 1, 0, 6, false>;
+      kernel = half <= 2   ? skinny_kernel<1, 1, 0, 2, true, false>
+               : half <= 3 ? skinny_kernel<1, 1, 0, 3, true, false>
+               : half <= 4 ? skinny_kernel<1, 1, 0, 4, true, false>
+               : waste(half, 4) <= waste(half, 3) ? skinny_kernel<1, 1, 0, 4, true, true> : skinny_kernel<1, 1, 0, 3, true, true>;
     else
-      kernel = a.M <= 16 ? skinny_kernel<1, 1, 0, 4, false> : skinny_kernel<2, 1, 0, 4, false>;
+      kernel = a.M <= 16 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
   } else {
-    kernel = a.M <= 16 ? skinny_kernel<1, CT, 0, 4, false> : skinny_kernel<2, CT, 0, 4, false>;
+    auto pick = [&](auto mt) {
+      constexpr int MT = decltype(mt)::value;
+      if constexpr (CT == 2) {
+        if (per <= 3) return skinny_kernel<MT, CT, 0, 3, false, false>;
+        if (per <= 4) return skinny_kernel<MT, CT, 0, 4, false, false>;
+      }
+      return skinny_kernel<MT, CT, 0, 4, false, true>;
+    };
+    kernel = a.M <= 16 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
   }
   kernel<<<grid, block, lds, st>>>(g);
   return launch_status("skinny_kernel");
@@ -678,8 +706,8 @@ extern "C" int lema_skinny_norm_qkv_bf16(const void* x, const void* nw, float ep
   if (int rc = qkv_args(a, ct, x, K, wq, wk, wv, ldw, M, Nqk, Nv, K, d, T, qcodes, kcodes,
                         code_bytes, v))
     return rc;
-  LEMA_REQUIRE(K <= 512 * kSkNormSteps, "the fused norm takes rows of at most %d elements, got K=%lld",
-               512 * kSkNormSteps, (long long)K);
+  LEMA_REQUIRE(K <= kSkNormMaxK, "the fused norm takes rows of at most %d elements, got K=%lld",
+               kSkNormMaxK, (long long)K);
   // LDS: the rows (M x (K + 8) bf16) next to the partial sums (8 x 16 or 32 rows x 16 ct + 1)
   const int64_t lds = M * (K + 8) * 2 + kSkWaves * (M <= 16 ? 16 : 32) * (16 * ct + 1) * 4;
   LEMA_REQUIRE(lds <= 160 * 1024, "%lld rows of %lld do not fit the LDS of a workgroup",
@@ -721,8 +749,8 @@ extern "C" int lema_skinny_norm_swiglu_bf16(const void* x, const void* d, const 
   if (int rc = check_weight(wg, N)) return rc;
   if (int rc = check_weight(wu, N)) return rc;
   LEMA_REQUIRE(out != nullptr, "bad output pointer");
-  LEMA_REQUIRE(K <= 512 * kSkNormSteps, "the fused norm takes rows of at most %d elements, got K=%lld",
-               512 * kSkNormSteps, (long long)K);
+  LEMA_REQUIRE(K <= kSkNormMaxK, "the fused norm takes rows of at most %d elements, got K=%lld",
+               kSkNormMaxK, (long long)K);
   // LDS: the rows (M x (K + 8) bf16) next to the partial sums (8 x 16 or 32 rows x 33 floats)
   const int64_t lds = M * (K + 8) * 2 + kSkWaves * (M <= 16 ? 16 : 32) * 33 * 4;
   LEMA_REQUIRE(lds <= 160 * 1024, "%lld rows of %lld do not fit the LDS of a workgroup",

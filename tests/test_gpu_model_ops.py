@@ -48,6 +48,21 @@ def test_rmsnorm_matches_torch(dev, residual):
     assert (h == want).float().mean() > 0.9999
 
 
+@pytest.mark.parametrize("D", [8, 512, 520, 1024, 1032, 1536, 1544, 2048, 2056, 4096])
+def test_rmsnorm_widths(dev, D):
+    """Rows of every number of steps that a kernel holds, from the shortest to the longest."""
+    norm = torch.nn.RMSNorm(D, eps=1e-5).to(dev).to(torch.bfloat16)
+    x, d = (torch.randn(37, D, device=dev).to(torch.bfloat16) for _ in range(2))
+    for add in (None, d):
+        with torch.no_grad():
+            h, xo = rms_norm(x, norm, add)
+        s = (x if add is None else x + d).double()
+        assert torch.equal(xo.double(), s)
+        want = s * torch.rsqrt(s.square().mean(-1, keepdim=True) + 1e-5) * norm.weight.double()
+        # one rounding to bf16, of a value that fp32 sums and products leave 2^-12 or less off
+        assert float(((h.double() - want).abs() - 2.0 ** -8 * (1 + 2.0 ** -4) * want.abs()).max()) <= 0.0
+
+
 def test_cross_entropy_from_bf16_logits(dev):
     V = 50304
     logits = (torch.randn(1000, V, device=dev) * 4).to(torch.bfloat16)
@@ -134,7 +149,7 @@ def test_device_copy(dev):
         _lib.check(_lib.lib().lema_device_copy(src.data_ptr(), dst.data_ptr(), 24, st))
 
 
-@pytest.mark.parametrize("V", [8, 8192, 65536 + 8, 70000])
+@pytest.mark.parametrize("V", [8, 8192, 8200, 16384, 20000, 32768, 32776, 65536 + 8, 70000])
 def test_argmax_signed_zeros_and_groups(dev, V):
     """-0 and +0 tie (the first wins), negative NaNs win too, and the maximum may lie in any
     group of pieces, the last piece of the row included."""

@@ -83,3 +83,33 @@ def test_code_bytes(dev, M, d, cb):
                                                 codes.data_ptr(), cb, _lib.stream_of(x)))
     got = codes.long() & 0xFFFFFFFF if cb == 4 else codes
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("K", [32, 256, 768, 800, 1024, 1056, 1536, 1568, 2048])
+@pytest.mark.parametrize("M", [1, 9, 17])
+@pytest.mark.parametrize("with_d", [False, True])
+def test_norm_shares(dev, K, M, with_d):
+    """A fused pre-norm's product at every size of its load group, each from its shortest to its
+    longest rows, against the norm in 64 bits and the product of its bf16 rows in fp32 sums."""
+    g = torch.Generator(device=dev).manual_seed(K + M)
+    x, d = (torch.randn((M, K), device=dev, generator=g).to(torch.bfloat16) for _ in range(2))
+    nw = (1 + 0.1 * torch.randn(K, device=dev, generator=g)).to(torch.bfloat16)
+    wg, wu = ((torch.randn((48, K), device=dev, generator=g) * K ** -0.5).to(torch.bfloat16) for _ in range(2))
+    out, h, xo = (torch.empty(s, device=dev, dtype=torch.bfloat16) for s in ((M, 48), (M, K), (M, K)))
+    L, st, dp = _lib.lib(), _lib.stream_of(x), d.data_ptr() if with_d else None
+    _lib.check(L.lema_skinny_norm_swiglu_bf16(x.data_ptr(), dp, nw.data_ptr(), 1e-5, xo.data_ptr(), wg.data_ptr(),
+                                              wu.data_ptr(), K, M, 48, K, out.data_ptr(), st))
+    _lib.check(L.lema_rmsnorm_bf16(x.data_ptr(), dp, nw.data_ptr(), 1e-5, M, K, xo.data_ptr() if with_d else None,
+                                   h.data_ptr(), st))
+    s = (x + d if with_d else x).double()
+    want_h = s * torch.rsqrt(s.square().mean(-1, keepdim=True) + 1e-5) * nw.double()
+    assert float((h.double() - want_h).abs().sub(2.0 ** -8 * want_h.abs() * (1 + 2.0 ** -12)).max()) <= 0.0
+    want = torch.empty_like(out)
+    _lib.check(L.lema_skinny_swiglu_bf16(h.data_ptr(), K, wg.data_ptr(), wu.data_ptr(), K, M, 48, K,
+                                         want.data_ptr(), st))
+    assert torch.equal(out, want)      # the same rows, sums in the same order
+    gate, up = h.double() @ wg.double().T, h.double() @ wu.double().T
+    ref = torch.nn.functional.silu(gate) * up
+    # gate, up, the silu and the result each rounded to bf16; the silu's slope is at most 1.1
+    bound = 2.0 ** -8 * (1.1 * gate.abs() * up.abs() + 3.1 * ref.abs()) * 1.01 + 1e-6
+    assert float(((out.double() - ref).abs() - bound).max()) <= 0.0
