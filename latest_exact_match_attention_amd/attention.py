@@ -230,13 +230,15 @@ def _plain_grad(gy: torch.Tensor) -> bool:
     """Whether a backward may hand gy to the kernel: an ordinary device tensor whose own
     gradient nobody asks for. A graph of the backward (create_graph), forward mode, batched
     gradients and traced or otherwise wrapped tensors keep the tensor operations, which
-    compose with them or refuse them by themselves."""
+    compose with them or refuse them by themselves. So do deterministic algorithms: the kernel
+    adds a source row's gradients in the order its wavefronts list them."""
     ft = torch._C._functorch
     return (type(gy) is torch.Tensor and gy.is_cuda and gy.dtype in _lib.DTYPE_CODE
             and not torch.is_grad_enabled() and torch._C._len_torch_dispatch_stack() == 0
             and not ft.is_functorch_wrapped_tensor(gy) and not ft.is_legacy_batchedtensor(gy)
             and torch.autograd.forward_ad._current_level < 0
-            and not gy.is_neg() and not gy._is_zerotensor())
+            and not gy.is_neg() and not gy._is_zerotensor()
+            and not torch.are_deterministic_algorithms_enabled())
 
 
 class _LemaGather(torch.autograd.Function):

@@ -132,3 +132,24 @@ def test_other_backwards_keep_composing(dev):
     with torch.autograd.graph.save_on_cpu():
         y2 = lema.attention._LemaGather.apply(qc, qc, v)
     torch.testing.assert_close(torch.autograd.grad(y2, v, gs[2])[0], each[2])
+
+
+@pytest.mark.parametrize("kind", ["first", "few"])
+def test_deterministic_algorithms(dev, kind):
+    """Under the switch the gradient is the tensor operations' own, bit for bit, every time."""
+    N, T, dv = 2, 9001, 24
+    g = torch.Generator().manual_seed(7)
+    qc, kc = (c.view(1, N, T).to(dev) for c in _codes(kind, N, T, g))
+    v = torch.randn((1, N, T, dv), generator=g).to(dev).requires_grad_(True)
+    gy = torch.randn((1, N, T, dv), generator=g).to(dev)
+    y = lema.attention._LemaGather.apply(qc, kc, v)
+    src = lema.lema_from_codes(qc, kc, v.detach(), return_src=True)[1].long()
+    idx = src.clamp_min(0).unsqueeze(-1).expand(1, N, T, dv)
+    torch.use_deterministic_algorithms(True)
+    try:
+        want = torch.zeros_like(gy).scatter_add_(2, idx, gy * (src >= 0).unsqueeze(-1))
+        for _ in range(2):
+            (gv,) = torch.autograd.grad(y, v, gy, retain_graph=True)
+            assert torch.equal(gv, want)
+    finally:
+        torch.use_deterministic_algorithms(False)
