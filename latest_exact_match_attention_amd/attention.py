@@ -226,14 +226,16 @@ def _hard_z(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     return y, src
 
 
-def _plain_grad(gy: torch.Tensor) -> bool:
-    """Whether a backward may hand gy to the kernel: an ordinary device tensor whose own
-    gradient nobody asks for. A graph of the backward (create_graph), forward mode, batched
+def _plain_grad(gy: torch.Tensor, src: torch.Tensor) -> bool:
+    """Whether a backward may hand gy and the saved indices to the kernel: an ordinary device
+    tensor whose own gradient nobody asks for, and the indices as they were saved (a saved-tensor
+    hook may bring them back in another type or on another device). A graph of the backward (create_graph), forward mode, batched
     gradients and traced or otherwise wrapped tensors keep the tensor operations, which
     compose with them or refuse them by themselves. So do deterministic algorithms: the kernel
     adds a source row's gradients in the order its wavefronts list them."""
     ft = torch._C._functorch
-    return (type(gy) is torch.Tensor and gy.is_cuda and gy.dtype in _lib.DTYPE_CODE
+    return (type(gy) is torch.Tensor and type(src) is torch.Tensor and src.dtype is torch.int32
+            and src.device == gy.device and src.shape == gy.shape[:3] and gy.is_cuda and gy.dtype in _lib.DTYPE_CODE
             and not torch.is_grad_enabled() and torch._C._len_torch_dispatch_stack() == 0
             and not ft.is_functorch_wrapped_tensor(gy) and not ft.is_legacy_batchedtensor(gy)
             and torch.autograd.forward_ad._current_level < 0
@@ -258,7 +260,7 @@ class _LemaGather(torch.autograd.Function):
     def backward(ctx, gy):
         (src,) = ctx.saved_tensors
         B, H, T, dv = ctx.v_shape
-        if _plain_grad(gy):
+        if _plain_grad(gy, src):
             gy = gy if gy.stride(-1) == 1 or dv == 1 else gy.contiguous()
             gv = torch.empty((B, H, T, dv), dtype=gy.dtype, device=gy.device)
             _lib.check(_lib.lib().lema_gather_grad(

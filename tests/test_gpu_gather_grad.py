@@ -153,3 +153,17 @@ def test_deterministic_algorithms(dev, kind):
             assert torch.equal(gv, want)
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+@pytest.mark.parametrize("kept", [torch.int64, torch.int16])
+def test_indices_that_a_hook_keeps_in_another_type(dev, kept):
+    """Saved-tensor hooks may bring the indices back wider or narrower than they were saved."""
+    qc = torch.randint(0, 6, (1, 2, 900), device=dev)
+    v = torch.randn((1, 2, 900, 8), device=dev, requires_grad=True)
+    gy = torch.randn((1, 2, 900, 8), device=dev)
+    (want,) = torch.autograd.grad(lema.attention._LemaGather.apply(qc, qc, v), v, gy)
+    with torch.autograd.graph.saved_tensors_hooks(lambda x: x.to(kept), lambda x: x):
+        y = lema.attention._LemaGather.apply(qc, qc, v)
+    (got,) = torch.autograd.grad(y, v, gy)
+    # a row's sum in another order: fp32, at most 900 terms
+    torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4)
