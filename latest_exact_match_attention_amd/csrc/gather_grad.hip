@@ -16,7 +16,9 @@
 // Every row of gv is written once, zeros included. A list that fills up before the scan ends is
 // reduced at once and the rows then accumulate in gv (rounded once per list, in 16-bit types).
 // The scan reads O(T^2 / R) indices from L2, 4 bytes each: at T = 100,000 and R = 1024 about
-// 49 per index against the 48 to 256 bytes of its gy row.
+// 49 per index against the 48 to 256 bytes of its gy row. It counts 8192 indices behind one
+// barrier before it lists them: with two barriers for every batch or two of 1024, one row of
+// 131,072 positions (d_v 24 bf16) took 104 us where 39 are now.
 //
 // A missed query's row is multiplied by zero and added to source row 0: nothing, unless it holds
 // an infinity or NaN, which make that column of gv[row, 0] NaN. A second kernel reads the missed
@@ -34,11 +36,12 @@ namespace {
 
 constexpr int kGgThreads = 256;
 constexpr int kGgRows = 1024;            // most source rows per workgroup
-constexpr int kGgBatch = 4 * kGgThreads; // indices between two looks at the list's room
-// Entries of the list: room for a batch beyond the 1536 that a scan may hold before it has to
-// look, with every LDS array of 4 workgroups in a CU's 160 KB.
+constexpr int kGgBatch = 4 * kGgThreads; // indices of a 16-byte load by every thread
+// Entries of the list: a list that is reduced early has no room for a batch, so it holds over 1536;
+// every LDS array of 4 workgroups fits a CU's 160 KB.
 constexpr int kGgList = 2560;
 constexpr int kGgFlight = 8;             // gy rows in flight per group of lanes
+constexpr int kGgSpan = 8;               // batches of indices whose loads are issued together
 constexpr int kMissPositions = 256;      // positions per workgroup of the miss kernel
 
 struct GradArgs {
@@ -173,14 +176,14 @@ struct GradLds {
   uint16_t perm_j[kGgList];
   int32_t end[kGgRows];                  // counts, then cursors: where a source row's run ends
   int32_t wave_sum[kGgThreads / 64];
-  int32_t count;                         // entries listed
+  int32_t incoming[3];                   // entries that the current span of indices adds
 };
 // A run's first sum when its row began in an earlier run, [element][thread]: the list's storage,
 // dead once it is sorted.
 static_assert(sizeof(int32_t) * kGgList >= sizeof(float) * 8 * kGgThreads, "the runs' first sums");
 
 template <int DTYPE, int VEC>
-__global__ __launch_bounds__(kGgThreads) void gather_grad_kernel(GradArgs a) {
+__global__ __launch_bounds__(kGgThreads, 4) void gather_grad_kernel(GradArgs a) {
   typedef GgPiece<DTYPE, VEC> P;
   constexpr int E = P::kElems;
   __shared__ GradLds s;
@@ -198,9 +201,8 @@ __global__ __launch_bounds__(kGgThreads) void gather_grad_kernel(GradArgs a) {
 
   bool accumulate = false;  // gv's rows hold earlier lists' sums
   // Sort the listed queries by source row and add their gy rows up (all threads).
-  auto reduce_list = [&](bool last) {
+  auto reduce_list = [&](int n, bool last) {
     __syncthreads();
-    const int n = s.count;
     for (int x = t; x < kGgRows; x += kGgThreads) s.end[x] = 0;
     __syncthreads();
     for (int e = t; e < n; e += kGgThreads) atomicAdd(&s.end[s.list_j[e]], 1);
@@ -311,59 +313,107 @@ __global__ __launch_bounds__(kGgThreads) void gather_grad_kernel(GradArgs a) {
       }
       __syncthreads();
     }
-    if (t == 0) s.count = 0;
-    __syncthreads();
   };
 
-  if (t == 0) s.count = 0;
+  if (t < 3) s.incoming[t] = 0;
   __syncthreads();
-  const unsigned long long below = (1ull << lane) - 1ull;
-  int most = 0;  // the list holds at most this many entries (the same in every thread)
-  auto list_batch = [&](int64_t i0, const int32_t (&x)[4]) {
+  const uint32_t first_j = static_cast<uint32_t>(j0), n_j = static_cast<uint32_t>(rows);
+  auto in = [&](int32_t x) { return static_cast<uint32_t>(x) - first_j < n_j; };  // a miss is no row either
+  // four consecutive indices from i on, 16-byte aligned where they all lie in the row
+  auto load4 = [&](int64_t i, int32_t (&x)[4]) {
+    if (i >= 0 && i + 3 < a.T) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(src + i);
+      x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+    } else {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t j = static_cast<int64_t>(x[u]) - j0;
-      const bool in = j >= 0 && j < rows;  // x is -1 past the row's end
-      const unsigned long long bal = __ballot(in);
-      if (bal == 0) continue;
-      int base = 0;
-      if (lane == 0) base = atomicAdd(&s.count, __popcll(bal));
-      base = __shfl(base, 0);
-      if (in) {
-        const int p = base + __popcll(bal & below);
-        s.list_i[p] = static_cast<int32_t>(i0 + u * kGgThreads + t);
-        s.list_j[p] = static_cast<uint16_t>(j);
+      for (int u = 0; u < 4; ++u) x[u] = i + u >= 0 && i + u < a.T ? src[i + u] : -1;
+    }
+  };
+  // bit 4q + u: x[q][u] points into the rows
+  auto mask_of = [&](const auto& x) {
+    constexpr int Q = sizeof(x) / sizeof(x[0]);
+    static_assert(4 * Q <= 32, "a bit each");
+    uint32_t m = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) m |= in(x[q][u]) ? 1u << (4 * q + u) : 0u;
+    return m;
+  };
+  // The list's places of the indices of mask m: `before` those of the threads ahead of this one, in
+  // all threads together `all`. A wavefront's places follow its turn at the counter, a thread's
+  // those of the lanes below it.
+  int turn = 0;
+  auto places = [&](uint32_t m, int& before, int& all) {
+    const int c = __popc(m);
+    int inc = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(inc, o);
+      if (lane >= o) inc += up;
+    }
+    int old = 0;
+    if (lane == 63 && inc != 0) old = atomicAdd(&s.incoming[turn], inc);
+    before = __shfl(old, 63) + inc - c;
+    __syncthreads();
+    all = s.incoming[turn];
+    // the counter before this one: read before the last barrier, used after the next
+    if (t == 0) s.incoming[turn == 0 ? 2 : turn - 1] = 0;
+    turn = turn == 2 ? 0 : turn + 1;
+  };
+  auto list = [&](int64_t i0, const auto& x, uint32_t m, int p) {
+    constexpr int Q = sizeof(x) / sizeof(x[0]);
+    if (m == 0) return;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (m >> (4 * q + u) & 1u) {
+          s.list_i[p] = static_cast<int32_t>(i0 + q * kGgBatch + 4 * t + u);
+          s.list_j[p] = static_cast<uint16_t>(x[q][u] - static_cast<int32_t>(j0));
+          ++p;
+        }
+  };
+  // A span of indices is counted before it is listed, so one barrier tells whether it fits; one
+  // that does not is listed by batches as far as there is room. (With a look at the list's
+  // room for every batch or two, rows of 131,072 spent most of the scan in barriers.) Indices
+  // at or before the first source row read rows below it, so the scan may begin up to three
+  // early, on a 16-byte boundary.
+  const int skew = static_cast<int>((reinterpret_cast<uintptr_t>(src + j0 + 1) & 15) / 4);
+  int64_t i0 = j0 + 1 - skew;
+  int listed = 0;  // entries of the list
+  bool full;
+  do {
+    full = false;
+    while (!full && i0 < a.T) {
+      int32_t x[kGgSpan][4];
+#pragma unroll
+      for (int q = 0; q < kGgSpan; ++q) load4(i0 + q * kGgBatch + 4 * t, x[q]);
+      const uint32_t m = mask_of(x);
+      int before, more;
+      places(m, before, more);
+      if (listed + more <= kGgList) {
+        list(i0, x, m, listed + before);
+        listed += more;
+        i0 += kGgSpan * kGgBatch;
+        continue;
       }
-    }
-  };
-  auto load_batch = [&](int64_t i0, int32_t (&x)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t i = i0 + u * kGgThreads + t;
-      x[u] = i < a.T ? src[i] : -1;
-    }
-  };
-  for (int64_t i0 = j0 + 1; i0 < a.T; i0 += 4 * kGgBatch) {
-    int32_t x[4][4];  // four batches' loads issued together
-#pragma unroll
-    for (int q = 0; q < 4; ++q) load_batch(i0 + q * kGgBatch, x[q]);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (i0 + q * kGgBatch >= a.T) break;
-      if (most > kGgList - kGgBatch) {  // the count itself, once the bound leaves no room
-        __syncthreads();
-        most = s.count;
-        __syncthreads();
-        if (most > kGgList - kGgBatch) {
-          reduce_list(false);
-          most = 0;
+      for (int q = 0; q < kGgSpan && !full && i0 < a.T; ++q) {
+        int32_t y[1][4];
+        load4(i0 + 4 * t, y[0]);
+        const uint32_t my = mask_of(y);
+        places(my, before, more);
+        full = listed + more > kGgList;
+        if (!full) {
+          list(i0, y, my, listed + before);
+          listed += more;
+          i0 += kGgBatch;
         }
       }
-      list_batch(i0 + q * kGgBatch, x[q]);
-      most += kGgBatch;
     }
-  }
-  reduce_list(true);
+    reduce_list(listed, !full);
+    listed = 0;
+  } while (full);
 }
 
 // Missed queries: an infinity or NaN in such a row of gy makes its column of gv[row, 0] NaN
