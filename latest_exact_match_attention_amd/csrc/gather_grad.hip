@@ -26,7 +26,7 @@
 //
 // Measured (MI355X), B2 H64 T8001 d_v 24 bf16 on projection views: 43 us and 17 us for the missed
 // rows (48.8 and 18.7 with each row of streams on its own XCD), against 590 us for the tensor
-// operations; B1 H8 T4096 d_v 64 fp32: 10.8 and 4.2 us against 88.
+// operations; B1 H8 T4096 d_v 64 fp32: 12.0 and 4.0 us against 88.
 #include "lema_internal.h"
 
 #include <hip/hip_fp16.h>
@@ -41,6 +41,7 @@ constexpr int kGgBatch = 4 * kGgThreads; // indices of a 16-byte load by every t
 // every LDS array of 4 workgroups fits a CU's 160 KB.
 constexpr int kGgList = 2560;
 constexpr int kGgFlight = 8;             // gy rows in flight per group of lanes
+constexpr int kGgSliceT = 16384;         // shorter rows' lists are short whoever reads what
 constexpr int kGgSpan = 8;               // batches of indices whose loads are issued together
 constexpr int kMissPositions = 256;      // positions per workgroup of the miss kernel
 
@@ -51,8 +52,9 @@ struct GradArgs {
   int64_t N, H, T;
   int64_t sb, sh, st;  // strides of gy, bytes
   int64_t row_bytes;
-  int32_t pieces;      // pieces per value row
-  int32_t R, nch;      // source rows per workgroup, workgroups per row
+  int32_t pieces;      // pieces per value row, or a slice of one
+  int32_t R, nch;      // source rows per workgroup, workgroups per row and slice
+  int32_t slices;      // slices of a value row's columns, a workgroup each
   int32_t order;       // of the workgroups (gg_item)
   FastDiv pdiv;        // division by `pieces`
 };
@@ -190,13 +192,14 @@ __global__ __launch_bounds__(kGgThreads, 4) void gather_grad_kernel(GradArgs a) 
   const int t = threadIdx.x, lane = t & 63;
   int64_t row;
   int part_no;
-  gg_item(a.order, a.N, a.nch, blockIdx.x, row, part_no);
-  const int64_t j0 = static_cast<int64_t>(part_no) * a.R;
+  gg_item(a.order, a.N, a.nch * a.slices, blockIdx.x, row, part_no);
+  const int64_t slice0 = static_cast<int64_t>(part_no % a.slices) * a.pieces * VEC;  // bytes
+  const int64_t j0 = static_cast<int64_t>(part_no / a.slices) * a.R;
   const int rows = static_cast<int>(a.T - j0 < a.R ? a.T - j0 : a.R);
   const int32_t* src = a.src + row * a.T;
   const int64_t b = row / a.H, h = row - (row / a.H) * a.H;
-  const uint8_t* gy = a.gy + b * a.sb + h * a.sh;
-  uint8_t* gv = a.gv + (row * a.T + j0) * a.row_bytes;
+  const uint8_t* gy = a.gy + b * a.sb + h * a.sh + slice0;
+  uint8_t* gv = a.gv + (row * a.T + j0) * a.row_bytes + slice0;
   float* part = reinterpret_cast<float*>(s.list_i);
 
   bool accumulate = false;  // gv's rows hold earlier lists' sums
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(kGgThreads, 4) void gather_grad_kernel(GradArgs a) 
       for (uint32_t x = t; x < static_cast<uint32_t>(rows) * a.pieces; x += kGgThreads) {
         const int j = static_cast<int>(a.pdiv.div(x));
         if (!last || s.end[j] == (j > 0 ? s.end[j - 1] : 0))
-          gg_store<VEC>(gv + static_cast<int64_t>(x) * VEC, zero);
+          gg_store<VEC>(gv + j * a.row_bytes + (x - static_cast<uint32_t>(j) * a.pieces) * VEC, zero);
       }
       if (!last) {
         accumulate = true;
@@ -469,17 +472,31 @@ __global__ __launch_bounds__(kGgThreads) void gather_grad_miss_kernel(GradArgs a
 
 template <int DTYPE, int VEC>
 int launch_grad(GradArgs& a, hipStream_t st) {
-  // Fewer source rows per workgroup while the launch has under 4 workgroups per CU
+  // While the launch has under 4 workgroups per CU: value rows in slices of at least 128 bytes (a
+  // workgroup lists and sorts for its slice alone, but where all queries read a few source rows it
+  // is one workgroup's loads that bound the launch: one row of 131,072 queries of the first
+  // 3 rows, d_v 64 fp32, 1420 us whole, 1016 in two slices), then fewer source rows.
+  const int32_t row_pieces = a.pieces;
+  const FastDiv row_pdiv = a.pdiv;
   a.R = kGgRows;
-  while (a.R > 64 && a.N * ((a.T + a.R - 1) / a.R) < 1024) a.R /= 2;
+  a.slices = 1;
+  auto few = [&] { return a.N * ((a.T + a.R - 1) / a.R) * a.slices < 1024; };
+  while (a.T >= kGgSliceT && a.pieces % 2 == 0 && a.pieces * VEC >= 256 && few()) {
+    a.slices *= 2;
+    a.pieces /= 2;
+  }
+  while (a.R > 64 && few()) a.R /= 2;
   const int64_t nch = (a.T + a.R - 1) / a.R;
   const int64_t mch = (a.T + kMissPositions - 1) / kMissPositions;
-  LEMA_REQUIRE(a.N < (int64_t(1) << 31) && a.N * mch < (int64_t(1) << 31) && a.N * nch < (int64_t(1) << 31),
+  LEMA_REQUIRE(a.N < (int64_t(1) << 31) && a.N * mch < (int64_t(1) << 31) && a.N * nch * a.slices < (int64_t(1) << 31),
                "too many rows x positions");
   a.nch = static_cast<int32_t>(nch);
+  a.pdiv = FastDiv(static_cast<uint32_t>(a.pieces));
   a.order = a.N % 64 == 0 ? kGgGroups : a.N % kNumXcd == 0 ? kGgRowXcd : kGgSpread;
-  gather_grad_kernel<DTYPE, VEC><<<dim3(a.N * nch), dim3(kGgThreads), 0, st>>>(a);
+  gather_grad_kernel<DTYPE, VEC><<<dim3(a.N * nch * a.slices), dim3(kGgThreads), 0, st>>>(a);
   if (int rc = launch_status("gather_grad_kernel")) return rc;
+  a.pieces = row_pieces;
+  a.pdiv = row_pdiv;
   gather_grad_miss_kernel<DTYPE, VEC>
       <<<dim3(a.N * mch), dim3(kGgThreads), 0, st>>>(a, static_cast<int32_t>(mch));
   return launch_status("gather_grad_miss_kernel");

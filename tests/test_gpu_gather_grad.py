@@ -62,6 +62,9 @@ def _view(x, form):
     # rows that don't fill the XCDs: their parts go round them
     ("few", 1, 1, 40001, 8, "plain"), ("many", 1, 7, 5003, 24, "projection"), ("spread", 3, 3, 2600, 16, "plain"),
     ("few", 1, 12, 1500, 24, "projection"), ("first", 1, 8, 2050, 8, "offset"),
+    # long enough for slices of the columns: 2, 4 and a row that none divides
+    ("few", 1, 1, 16384, 64, "plain"), ("first", 1, 2, 17000, 128, "projection"), ("many", 1, 1, 16400, 260, "plain"),
+    ("few", 1, 1, 16390, 65, "plain"),
 ])
 def test_gradient_is_the_sum(dev, dtype, kind, B, H, T, dv, form):
     g = torch.Generator().manual_seed(T + dv)
