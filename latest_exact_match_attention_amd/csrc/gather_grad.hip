@@ -485,7 +485,8 @@ int launch_grad(GradArgs& a, hipStream_t st) {
     a.slices *= 2;
     a.pieces /= 2;
   }
-  while (a.R > 64 && few()) a.R /= 2;
+  // and no more pieces than 32 bits count
+  while (a.R > 64 && (few() || static_cast<int64_t>(a.R) * a.pieces >= (int64_t(1) << 31))) a.R /= 2;
   const int64_t nch = (a.T + a.R - 1) / a.R;
   const int64_t mch = (a.T + kMissPositions - 1) / kMissPositions;
   LEMA_REQUIRE(a.N < (int64_t(1) << 31) && a.N * mch < (int64_t(1) << 31) && a.N * nch * a.slices < (int64_t(1) << 31),
@@ -529,7 +530,6 @@ extern "C" int lema_gather_grad(const void* gy, int32_t dtype, int64_t B, int64_
   LEMA_REQUIRE(B >= 0 && H >= 0 && T >= 0 && dv >= 0, "negative shape");
   if (B * H * T * dv == 0) return LEMA_OK;
   LEMA_REQUIRE(T < (int64_t(1) << 30), "T=%lld exceeds the resolver's positions", (long long)T);
-  LEMA_REQUIRE(dv < (int64_t(1) << 20), "value rows too long (%lld elements)", (long long)dv);
   LEMA_REQUIRE(gy != nullptr && src != nullptr && gv != nullptr && aligned(src, 4),
                "gy, src and gv must be device pointers");
   // the largest piece that divides the row and every offset of gy and gv
@@ -539,6 +539,8 @@ extern "C" int lema_gather_grad(const void* gy, int32_t dtype, int64_t B, int64_
                      !aligned(gy, vec) || !aligned(gv, vec)))
     vec /= 2;
   LEMA_REQUIRE(vec >= es, "gradient rows not aligned to the element size");
+  // the gather's rows have at most 2^20 pieces, of 16 bytes at most: 2^23 of 2 bytes
+  LEMA_REQUIRE(rb / vec <= (int64_t(1) << 23), "value rows too long (%lld elements)", (long long)dv);
   GradArgs a{};
   a.gy = static_cast<const uint8_t*>(gy);
   a.src = src;

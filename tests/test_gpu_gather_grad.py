@@ -170,3 +170,15 @@ def test_indices_that_a_hook_keeps_in_another_type(dev, kept):
     (got,) = torch.autograd.grad(y, v, gy)
     # a row's sum in another order: fp32, at most 900 terms
     torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4)
+
+
+def test_rows_as_wide_as_the_forward_takes(dev):
+    """Value rows of 2^20 and more elements have a gradient too, in pieces of 16 and of 4 bytes."""
+    dv = (1 << 20) + 8
+    for at in (0, 1):                                # gy's rows on and off a 16-byte boundary
+        qc = torch.zeros((1, 1, 3), dtype=torch.int32, device=dev)
+        v = torch.randn((1, 1, 3, dv), device=dev, requires_grad=True)
+        gy = torch.randn((1, 1, 3, dv + 4), device=dev)[..., at:at + dv]
+        (gv,) = torch.autograd.grad(lema.attention._LemaGather.apply(qc, qc, v), v, gy)
+        want = torch.stack([gy[0, 0, 1], gy[0, 0, 2], torch.zeros_like(gy[0, 0, 0])])
+        assert torch.equal(gv[0, 0], want), at       # query 1 reads row 0, query 2 row 1
