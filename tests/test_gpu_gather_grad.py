@@ -182,3 +182,21 @@ def test_rows_as_wide_as_the_forward_takes(dev):
         (gv,) = torch.autograd.grad(lema.attention._LemaGather.apply(qc, qc, v), v, gy)
         want = torch.stack([gy[0, 0, 1], gy[0, 0, 2], torch.zeros_like(gy[0, 0, 0])])
         assert torch.equal(gv[0, 0], want), at       # query 1 reads row 0, query 2 row 1
+
+
+def test_the_longest_rows_keep_the_tensor_operations(dev, monkeypatch):
+    """Rows from attention.GRAD_KERNEL_T on take the tensor operations, shorter ones the kernel."""
+    qc = torch.randint(0, 6, (1, 2, 300), device=dev)
+    v = torch.randn((1, 2, 300, 8), device=dev, requires_grad=True)
+    gy = torch.randn((1, 2, 300, 8), device=dev)
+    y = lema.attention._LemaGather.apply(qc, qc, v)
+    calls = []
+    check = lema.attention._lib.check
+    monkeypatch.setattr(lema.attention._lib, "check", lambda rc: (calls.append(rc), check(rc)))
+    both = []
+    for line, kernel in ((301, 1), (300, 0)):
+        monkeypatch.setattr(lema.attention, "GRAD_KERNEL_T", line)
+        calls.clear()
+        both.append(torch.autograd.grad(y, v, gy, retain_graph=True)[0])
+        assert len(calls) == kernel, line
+    torch.testing.assert_close(both[0], both[1], rtol=1e-4, atol=1e-4)  # sums in another order
