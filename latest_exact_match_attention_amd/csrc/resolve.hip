@@ -201,9 +201,9 @@ constexpr int kSummaryMinChunks = 64;
 template <typename CodeT>
 __global__ __launch_bounds__(kThreads) void summary_kernel(ResolveArgs a) {
   __shared__ __attribute__((aligned(16))) CodeT code[kSumSlots];  // read 4 slots at a time
-  __shared__ int32_t last[kSumSlots];
-  __shared__ __attribute__((aligned(16))) uint32_t bits[kMaskWords];
-  __shared__ int32_t sent_last, lone;
+  __shared__ __attribute__((aligned(16))) int32_t last[kSumSlots];  // then the chunk's code bits
+  static_assert(kSumSlots == kMaskWords, "the bits take the place of the positions");
+  __shared__ int32_t sent_last, lone_of[kThreads / 64];
   const int per = a.nchunks - 1;
   const int bid = blockIdx.x;
   const int xcd = bid % kNumXcd;
@@ -235,18 +235,20 @@ __global__ __launch_bounds__(kThreads) void summary_kernel(ResolveArgs a) {
       kk[p] = krow[o[p]];
     }
   }
-  for (int x = t; x < kSumSlots; x += kThreads) {
-    code[x] = SENT;
-    last[x] = -1;
+  {  // both tables start as all ones
+    const u32x4 ones = {~0u, ~0u, ~0u, ~0u};
+    u32x4* c16 = reinterpret_cast<u32x4*>(code);
+    u32x4* l16 = reinterpret_cast<u32x4*>(last);
+    for (int x = t; x < kSumSlots * static_cast<int>(sizeof(CodeT)) / 16; x += kThreads) c16[x] = ones;
+    for (int x = t; x < kSumSlots / 4; x += kThreads) l16[x] = ones;
   }
-  for (int x = t; x < kMaskWords; x += kThreads) bits[x] = 0;
-  if (t == 0) {
-    sent_last = -1;
-    lone = 0;
-  }
-  // every fourth query of the chunk, to see how many have no key in it
-  static_assert(kLoneSample == kThreads, "a query per thread");
-  const CodeT q = (static_cast<const CodeT*>(a.qc) + row * a.T + chunk * kChunk)[kPer * t];
+  if (t == 0) sent_last = -1;
+  // a quarter of the chunk's queries, another quarter in the next chunk, to see how many have no
+  // key in it (spread over the chunk they touched every line of the queries: 3 us of 24 rows x
+  // T = 262144)
+  static_assert(kLoneSample == kThreads && kChunk == 4 * kThreads, "a query per thread");
+  const CodeT q = (static_cast<const CodeT*>(a.qc) + row * a.T + chunk * kChunk)[(chunk & 3) * kThreads + t];
+  uint32_t fresh = 0;  // bit p: this thread put kk[p] into the table
   __syncthreads();
 #pragma unroll
   for (int p = 0; p < kPer; ++p) {
@@ -257,10 +259,7 @@ __global__ __launch_bounds__(kThreads) void summary_kernel(ResolveArgs a) {
     bool ins;
     const int sl = table_claim<CodeT, kSumBuckets>(code, kk[p], SENT, bucket_of<kSumBuckets>(fold(kk[p])), ins);
     atomicMax(&last[sl], o[p]);
-    if (ins) {
-      const uint32_t h = mask_hash(fold(kk[p]));
-      atomicOr(&bits[h >> 5], 1u << (h & 31));
-    }
+    fresh |= ins ? 1u << p : 0u;
   }
   __syncthreads();
   {
@@ -269,15 +268,7 @@ __global__ __launch_bounds__(kThreads) void summary_kernel(ResolveArgs a) {
     read_bucket(code, b, x);
     const bool none = q != SENT && table_find<CodeT, kSumBuckets>(code, q, SENT, b, x) < 0;
     const int n = __popcll(__ballot(none));
-    if ((t & 63) == 0 && n) atomicAdd(&lone, n);
-  }
-  __syncthreads();
-  const int64_t rc = row * a.nchunks + chunk;
-  if (t == 0) a.summ_lone[rc] = static_cast<uint16_t>(lone);
-  if (lone > kLoneChunk && (lone <= kLoneQueue || a.nchunks > kMaskQueueChunks)) {
-    uint32_t* out_bits = a.summ_bits + rc * kMaskWords;
-    for (int x = t; x < kMaskWords / 4; x += kThreads)
-      *reinterpret_cast<u32x4*>(out_bits + 4 * x) = *reinterpret_cast<const u32x4*>(bits + 4 * x);
+    if ((t & 63) == 0) lone_of[t >> 6] = n;
   }
   uint32_t* tab = a.summ_tab + (row * a.nchunks + chunk) * kSumSlots;
   for (int b = t; b < kSumBuckets; b += kThreads) {
@@ -291,16 +282,42 @@ __global__ __launch_bounds__(kThreads) void summary_kernel(ResolveArgs a) {
     *reinterpret_cast<u32x4*>(tab + 4 * b) = u32x4{e[0], e[1], e[2], e[3]};
   }
   if (t == 0) a.summ_sent[row * a.nchunks + chunk] = sent_last;
+  __syncthreads();
+  // The bits only where the row may want them: made with the table they cost every row of few
+  // codes (24 x T = 262144 over 600 values: this kernel 33.7 us, 29.6 now, 24.1 without the sample
+  // and the bits; over 16 values 20.5, 18.9 and 17.6).
+  const int64_t rc = row * a.nchunks + chunk;
+  int lone = 0;
+#pragma unroll
+  for (int w = 0; w < kThreads / 64; ++w) lone += lone_of[w];
+  if (t == 0) a.summ_lone[rc] = static_cast<uint16_t>(lone);
+  if (lone > kLoneChunk && (lone <= kLoneQueue || a.nchunks > kMaskQueueChunks)) {
+    uint32_t* bits = reinterpret_cast<uint32_t*>(last);
+    for (int x = t; x < kMaskWords; x += kThreads) bits[x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < kPer; ++p)
+      if (fresh >> p & 1u) {
+        const uint32_t h = mask_hash(fold(kk[p]));
+        atomicOr(&bits[h >> 5], 1u << (h & 31));
+      }
+    __syncthreads();
+    uint32_t* out_bits = a.summ_bits + rc * kMaskWords;
+    for (int x = t; x < kMaskWords / 4; x += kThreads)
+      *reinterpret_cast<u32x4*>(out_bits + 4 * x) = *reinterpret_cast<const u32x4*>(bits + 4 * x);
+  }
 }
 
 // The chunks' code bits turned round: from one run of 65,536 bits per chunk to one run of
 // nchunks bits per code hash. A wavefront takes 64 chunks (one per lane) x kTurnWords 64-bit
 // words and transposes each 64 x 64 block with six exchanges between lanes; the wavefronts of
-// a workgroup take the row's 64-chunk blocks, whose words of a hash are adjacent.
+// a workgroup take the row's 64-chunk blocks, whose words of a hash are adjacent. Bound by the
+// round trips of a wavefront: with 4 runs of kTurnWords one after another and the wavefronts past
+// the row's blocks idle it took 20.5 us for 24 rows x T = 100003, 14.4 now.
 constexpr int kTurnWords = 8;
-constexpr int kTurnTrips = 4;  // runs of kTurnWords per workgroup, one after another
+constexpr int kTurnRuns = 2;  // runs of kTurnWords per workgroup, a wavefront each
 __global__ __launch_bounds__(kThreads) void mask_kernel(ResolveArgs a) {
-  constexpr int kParts = kMaskWords / 2 / (kTurnWords * kTurnTrips);
+  constexpr int kParts = kMaskWords / 2 / (kTurnWords * kTurnRuns);
   // the bits whose index has bit s clear
   constexpr uint64_t kLow[6] = {0x5555555555555555ull, 0x3333333333333333ull, 0x0F0F0F0F0F0F0F0Full,
                                 0x00FF00FF00FF00FFull, 0x0000FFFF0000FFFFull, 0x00000000FFFFFFFFull};
@@ -312,39 +329,43 @@ __global__ __launch_bounds__(kThreads) void mask_kernel(ResolveArgs a) {
   const int lane = threadIdx.x & 63;
   const int full = a.nchunks - 1;  // the row's last chunk has no summary
   const uint16_t* lone = a.summ_lone + row * a.nchunks;
-  int64_t sum = 0;  // of the row's samples, in every wavefront
-  for (int c = lane; c < full; c += 64) sum += lone[c];
+  int sum = 0;  // of the row's samples (under 2^20 chunks), in every wavefront
+  for (int c0 = lane; c0 < full; c0 += 8 * 64) {
+    int n[8];
 #pragma unroll
-  for (int s = 32; s > 0; s >>= 1) sum += __shfl_xor(static_cast<long long>(sum), s);
-  const bool built = sum > static_cast<int64_t>(kLoneRow) * full &&
-                     !(a.nchunks <= kMaskQueueChunks && sum > static_cast<int64_t>(kLoneQueue) * full);
+    for (int i = 0; i < 8; ++i) n[i] = c0 + 64 * i < full ? lone[c0 + 64 * i] : 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum += n[i];
+  }
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) sum += __shfl_xor(sum, s);
+  const bool built = sum > kLoneRow * full && !(a.nchunks <= kMaskQueueChunks && sum > kLoneQueue * full);
   if (part == 0 && threadIdx.x == 0) a.mask_built[row] = built;
   if (!built) return;
-  for (int cb = threadIdx.x >> 6; cb < a.mask_words; cb += kThreads / 64) {
+  for (int item = threadIdx.x >> 6; item < a.mask_words * kTurnRuns; item += kThreads / 64) {
+    const int cb = item / kTurnRuns;
+    const int w0 = (part * kTurnRuns + item % kTurnRuns) * kTurnWords;
     const int64_t chunk = 64 * cb + lane;
     const int ln = chunk < full ? lone[chunk] : 0;
     const bool have = ln > kLoneChunk && (ln <= kLoneQueue || a.nchunks > kMaskQueueChunks);  // as summary_kernel
-    for (int w0 = part * kTurnTrips * kTurnWords; w0 < (part + 1) * kTurnTrips * kTurnWords; w0 += kTurnWords) {
-      uint64_t x[kTurnWords];
+    uint64_t x[kTurnWords];
 #pragma unroll
-      for (int i = 0; i < kTurnWords; ++i) x[i] = chunk < full ? ~0ull : 0;
-      if (have) {
-        const uint64_t* p =
-            reinterpret_cast<const uint64_t*>(a.summ_bits + (row * a.nchunks + chunk) * kMaskWords) + w0;
+    for (int i = 0; i < kTurnWords; ++i) x[i] = chunk < full ? ~0ull : 0;
+    if (have) {
+      const uint64_t* p = reinterpret_cast<const uint64_t*>(a.summ_bits + (row * a.nchunks + chunk) * kMaskWords) + w0;
 #pragma unroll
-        for (int i = 0; i < kTurnWords; ++i) x[i] = p[i];
+      for (int i = 0; i < kTurnWords; ++i) x[i] = p[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kTurnWords; ++i) {
+      uint64_t v = x[i];
+#pragma unroll
+      for (int s = 5; s >= 0; --s) {
+        const int j = 1 << s;
+        const uint64_t y = __shfl_xor(static_cast<unsigned long long>(v), j);
+        v = (lane & j) ? ((v & ~kLow[s]) | ((y >> j) & kLow[s])) : ((v & kLow[s]) | ((y & kLow[s]) << j));
       }
-#pragma unroll
-      for (int i = 0; i < kTurnWords; ++i) {
-        uint64_t v = x[i];
-#pragma unroll
-        for (int s = 5; s >= 0; --s) {
-          const int j = 1 << s;
-          const uint64_t y = __shfl_xor(static_cast<unsigned long long>(v), j);
-          v = (lane & j) ? ((v & ~kLow[s]) | ((y >> j) & kLow[s])) : ((v & kLow[s]) | ((y & kLow[s]) << j));
-        }
-        a.summ_mask[((row << kMaskLog2) + 64 * (w0 + i) + lane) * a.mask_words + cb] = v;
-      }
+      a.summ_mask[((row << kMaskLog2) + 64 * (w0 + i) + lane) * a.mask_words + cb] = v;
     }
   }
 }
@@ -463,7 +484,7 @@ int launch_resolve(ResolveArgs& a, int vec, hipStream_t st) {
     const int64_t sgrid = (a.N + kNumXcd - 1) / kNumXcd * kNumXcd * (a.nchunks - 1);
     summary_kernel<CodeT><<<dim3(sgrid), dim3(kThreads), 0, st>>>(a);
     if (int rc = launch_status("summary_kernel")) return rc;
-    const int64_t mgrid = (a.N + kNumXcd - 1) / kNumXcd * kNumXcd * (kMaskWords / 2 / (kTurnWords * kTurnTrips));
+    const int64_t mgrid = (a.N + kNumXcd - 1) / kNumXcd * kNumXcd * (kMaskWords / 2 / (kTurnWords * kTurnRuns));
     LEMA_REQUIRE(mgrid < (int64_t(1) << 31), "too many rows (%lld)", (long long)a.N);
     mask_kernel<<<dim3(mgrid), dim3(kThreads), 0, st>>>(a);
     if (int rc = launch_status("mask_kernel")) return rc;

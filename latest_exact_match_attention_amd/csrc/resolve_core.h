@@ -322,8 +322,49 @@ constexpr int kMaskWords = (1 << kMaskLog2) / 32;  // summ_bits words per chunk
 // queued scan instead (32 rows x T = 65536 of uniform codes: 105 us without bits, 121 with).
 constexpr int kLoneSample = 256, kLoneRow = 56, kLoneChunk = 52, kLoneQueue = 230;
 constexpr int kMaskQueueChunks = 72;
+// The first step of the MurmurHash3 32-bit finaliser, top bits.
 __device__ __forceinline__ uint32_t mask_hash(uint32_t h) {
-  return ((h ^ (h >> 15)) * 0x2C1B3C6Du) >> (32 - kMaskLog2);
+  return ((h ^ (h >> 16)) * 0x85EBCA6Bu) >> (32 - kMaskLog2);
+}
+
+// before_chunk with the code's run of chunk bits `mask`; tab and krow are the row's summaries and
+// keys. A function of its own: inlined, its registers cost rows that have no bits 2 to 3 us of the
+// resolver (24 rows x T = 262144 over 16 codes: 69.4 us, 67.8 now, 67.0 without the bits' side; over
+// 600: 143.7, 141.1 and 141.2).
+template <typename CodeT>
+__device__ __attribute__((noinline)) int32_t masked_lookup(const uint32_t* tab, const CodeT* krow,
+                                                           const uint64_t* mask, int chunk, CodeT x) {
+  const uint32_t fp = fingerprint(fold(x));
+  const int b0 = bucket_of<kSumBuckets>(fold(x));
+  int wi = (chunk - 1) >> 6;
+  uint64_t cur = mask[wi] & (~0ull >> (63 - ((chunk - 1) & 63)));
+  uint64_t nxt = wi > 0 ? mask[wi - 1] : 0;  // read ahead of its use
+  constexpr int kTry = 4;
+  for (;;) {
+    int cc[kTry];
+    u32x4 e[kTry];
+#pragma unroll
+    for (int i = 0; i < kTry; ++i) {
+      while (cur == 0 && wi > 0) {
+        --wi;
+        cur = nxt;
+        nxt = wi > 0 ? mask[wi - 1] : 0;
+      }
+      cc[i] = -1;
+      if (cur != 0) {
+        const int b = 63 - __clzll(cur);
+        cur ^= 1ull << b;
+        cc[i] = (wi << 6) + b;
+        e[i] = *reinterpret_cast<const u32x4*>(tab + static_cast<int64_t>(cc[i]) * kSumSlots + 4 * b0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kTry; ++i) {
+      if (cc[i] < 0) return -1;
+      const int32_t j = summary_probe(tab + static_cast<int64_t>(cc[i]) * kSumSlots, krow, cc[i], x, fp, b0, e[i]);
+      if (j >= 0) return j;
+    }
+  }
 }
 
 // Latest key position before chunk `chunk` of row `row` for code x (sent: x is the all-ones
@@ -366,36 +407,8 @@ __device__ __forceinline__ int32_t before_chunk(const ResolveArgs& a, int64_t ro
     }
     return -1;
   }
-  const uint64_t* mask = a.summ_mask + ((row << kMaskLog2) + mask_hash(fold(x))) * a.mask_words;
-  int wi = (chunk - 1) >> 6;
-  uint64_t cur = mask[wi] & (~0ull >> (63 - ((chunk - 1) & 63)));
-  uint64_t nxt = wi > 0 ? mask[wi - 1] : 0;  // read ahead of its use
-  constexpr int kTry = 4;
-  for (;;) {
-    int cc[kTry];
-    u32x4 e[kTry];
-#pragma unroll
-    for (int i = 0; i < kTry; ++i) {
-      while (cur == 0 && wi > 0) {
-        --wi;
-        cur = nxt;
-        nxt = wi > 0 ? mask[wi - 1] : 0;
-      }
-      cc[i] = -1;
-      if (cur != 0) {
-        const int b = 63 - __clzll(cur);
-        cur ^= 1ull << b;
-        cc[i] = (wi << 6) + b;
-        e[i] = *reinterpret_cast<const u32x4*>(a.summ_tab + (rc + cc[i]) * kSumSlots + 4 * b0);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kTry; ++i) {
-      if (cc[i] < 0) return -1;
-      const int32_t j = summary_probe(a.summ_tab + (rc + cc[i]) * kSumSlots, krow, cc[i], x, fp, b0, e[i]);
-      if (j >= 0) return j;
-    }
-  }
+  return masked_lookup<CodeT>(a.summ_tab + rc * kSumSlots, krow,
+                              a.summ_mask + ((row << kMaskLog2) + mask_hash(fold(x))) * a.mask_words, chunk, x);
 }
 
 // ------------------------------------------------------------------ miss fill (dense path)
@@ -643,6 +656,8 @@ __device__ __forceinline__ void resolve_chunk(ResolveLds<CodeT>& s, const Resolv
     q[p] = act[p] ? qrow[c0 + o] : CodeT(0);
     kk[p] = act[p] ? krow[c0 + o] : CodeT(0);
   }
+  bool masked = false;  // read here: its latency is no part of the look-up's
+  if constexpr (kSumm) masked = a.mask_built[row] != 0;
   // Keys before the chunk stream in batches of 1024 (4 per thread), latest batch first, the
   // next kPrefetch batches loaded while the current one is looked up; c0 is a multiple of the
   // batch.
@@ -1015,7 +1030,6 @@ __device__ __forceinline__ void resolve_chunk(ResolveLds<CodeT>& s, const Resolv
         if (s.pos[x] == -2) need[atomicAdd(&s.nneed, 1)] = x;
       bar();
       const int nneed = s.nneed;
-      const bool masked = a.mask_built[row] != 0;
       for (int i = t; i < nneed; i += kThreads) {
         const int x = need[i];
         s.pos[x] = before_chunk<CodeT>(a, row, chunk, x == kSlots ? SENT : s.code[x], x == kSlots,
@@ -1041,7 +1055,7 @@ __device__ __forceinline__ void resolve_chunk(ResolveLds<CodeT>& s, const Resolv
   if (!filt) {
     rest(std::false_type{}, std::false_type{});
   } else if constexpr (kSumm) {
-    if (s.nq > kQueueSummMinCodes && (chunk < kQueueSummChunks || a.mask_built[row] == 0))
+    if (s.nq > kQueueSummMinCodes && (chunk < kQueueSummChunks || !masked))
       rest(std::true_type{}, std::true_type{});
     else
       rest(std::true_type{}, std::false_type{});
