@@ -58,7 +58,7 @@ def test_rmsnorm_widths(dev, D):
             h, xo = rms_norm(x, norm, add)
         s = (x if add is None else x + d).double()
         assert torch.equal(xo.double(), s)
-        want = s * torch.rsqrt(s.square().mean(-1, keepdim=True) + 1e-5) * norm.weight.double()
+        want = s * torch.rsqrt(s.square().mean(-1, keepdim=True) + 1e-5) * norm.weight.detach().double()
         # one rounding to bf16, of a value that fp32 sums and products leave 2^-12 or less off
         assert float(((h.double() - want).abs() - 2.0 ** -8 * (1 + 2.0 ** -4) * want.abs()).max()) <= 0.0
 
