@@ -87,10 +87,11 @@ struct SkDevice {
   const uint16_t* w;
   void* out;
   const uint16_t* add;   // plain: the residual or null; pre-norm: the addend or null
-  uint32_t ldx8, ldw8;   // row strides of x and the weights, in 8 elements
+  uint32_t ldx8, ldw8;   // row strides of x and the weights, in 8 elements: their low 32 bits
   int32_t K, N;
   int64_t ldy;
   uint32_t flags;        // mode | segments << 2 | code bytes << 4 | columns per block << 8 | M << 16
+                         // | the strides' next 5 bits << 22 (x) and << 27 (weights)
   int32_t blocks;        // of the first segment, and of the second
   const uint16_t* w1;    // the second segment's, or swiglu's up
   const uint16_t* w2;    // the third segment's: plain, Nv columns
@@ -137,7 +138,7 @@ __device__ __forceinline__ u32x4 swap_halves(u32x4 v) {
 // for K of up to 768, 1024, 1536 or 2048), and the weights' loads are issued before the
 // pre-norm's arithmetic and arrive meanwhile. Steps past the share cost a load each, and a second
 // group's registers keep other workgroups off the CU: K = 768, N = 50304 (3 steps) took
-// 22.6 us at M = 1 and 42.6 at M = 17 with groups of 4 and room for two, NEW1 and NEW17 now
+// 22.6 us at M = 1 and 42.6 at M = 17 with groups of 4 and room for two, 14.8 and 24.4 now
 // (16.4 and 27.4 with every load conditional).
 //
 // kHalf: a narrow block (8 columns) of at most 8 rows loads a second K-step into the matrix
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
   static_assert(!kHalf || (MT == 1 && CT == 1 && kNorm == 0), "a half-filled tile");
   __shared__ float part[kSkWaves][MT * 16][CT * 16 + 1];
   extern __shared__ __align__(16) uint16_t xs[];  // kNorm: the normalised rows, stride K + 8
-  const int M = a.flags >> 16, cols = (a.flags >> 8) & 0xFF, code_bytes = (a.flags >> 4) & 0xF;
+  const int M = (a.flags >> 16) & 0x3F, cols = (a.flags >> 8) & 0xFF, code_bytes = (a.flags >> 4) & 0xF;
   int mode = a.flags & 3, N = a.N, bid = blockIdx.x;
   const uint16_t* wbase = a.w;
   void* dst = a.out;
@@ -173,7 +174,8 @@ __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 
   }
   const bool glu = mode == kSkSwiglu;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
-  const int64_t ldx = static_cast<int64_t>(a.ldx8) * 8, ldw = static_cast<int64_t>(a.ldw8) * 8;
+  const int64_t ldx = (static_cast<int64_t>((a.flags >> 22) & 31) << 32 | a.ldx8) * 8;
+  const int64_t ldw = (static_cast<int64_t>(a.flags >> 27) << 32 | a.ldw8) * 8;
   const int n0 = bid * cols;
   const int ksteps = a.K / 32;
   const int per = (ksteps + kSkWaves - 1) / kSkWaves;
@@ -457,15 +459,16 @@ int launch_skinny(SkinnyArgs& a, hipStream_t st) {
   g.w = s0.w;
   g.out = s0.out;
   g.add = a.nw != nullptr ? a.nd : s0.res;
-  // the stride of a single row is never used
-  g.ldx8 = static_cast<uint32_t>((a.M > 1 ? a.ldx : a.K) / 8);
+  // 37 bits hold any stride that has a second row in memory; that of a single row is never used
+  g.ldx8 = static_cast<uint32_t>(a.ldx / 8);
   g.ldw8 = static_cast<uint32_t>(a.ldw / 8);
   g.K = a.K;
   g.N = s0.N;
   g.ldy = a.nseg == 3 ? a.seg[2].ldy : s0.ldy;
   g.flags = static_cast<uint32_t>(s0.mode) | static_cast<uint32_t>(a.nseg) << 2 |
             static_cast<uint32_t>(s0.code_bytes) << 4 | static_cast<uint32_t>(cols) << 8 |
-            static_cast<uint32_t>(a.M) << 16;
+            static_cast<uint32_t>(a.M) << 16 | static_cast<uint32_t>(a.ldx >> 35 & 31) << 22 |
+            static_cast<uint32_t>(a.ldw >> 35 & 31) << 27;
   g.blocks = (s0.N + cols - 1) / cols;
   g.w1 = a.nseg == 3 ? a.seg[1].w : s0.w2;
   g.w2 = a.seg[2].w;
@@ -542,7 +545,6 @@ int check_skinny(const void* x, int64_t ldx, int64_t ldw, int64_t M, int64_t K) 
                (long long)K);
   LEMA_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0,
                "row strides must be >= K and multiples of 8");
-  LEMA_REQUIRE((M == 1 || ldx < (int64_t(1) << 34)) && ldw < (int64_t(1) << 34), "row strides past 2^34 elements");
   LEMA_REQUIRE(x != nullptr && aligned(x, 16), "x must be a 16-byte aligned device pointer");
   return LEMA_OK;
 }

@@ -113,3 +113,19 @@ def test_norm_shares(dev, K, M, with_d):
     # gate, up, the silu and the result each rounded to bf16; the silu's slope is at most 1.1
     bound = 2.0 ** -8 * (1.1 * gate.abs() * up.abs() + 3.1 * ref.abs()) * 1.01 + 1e-6
     assert float(((out.double() - ref).abs() - bound).max()) <= 0.0
+
+
+def test_rows_far_apart(dev):
+    """Row strides past 2^35 elements: two rows of x, and two of a weight, 64 GiB apart."""
+    ld, K = (1 << 35) + 8, 64
+    if torch.cuda.mem_get_info(dev)[0] < 2 * ld + (8 << 30):
+        pytest.skip("needs 72 GiB of free memory")
+    far = torch.empty(ld + K, dtype=torch.bfloat16, device=dev)
+    rows = torch.randn((2, K), device=dev).to(torch.bfloat16)
+    far[:K], far[ld:] = rows[0], rows[1]
+    near = torch.randn((2, K), device=dev).to(torch.bfloat16)
+    y = torch.empty((2, 2), dtype=torch.bfloat16, device=dev)
+    for x, w, ldx, ldw, want in ((far, near, ld, K, _product(rows, near)), (near, far, K, ld, _product(near, rows))):
+        _lib.check(_lib.lib().lema_skinny_gemm_bf16(x.data_ptr(), ldx, w.data_ptr(), ldw, y.data_ptr(), 2, 2, 2, K,
+                                                    _lib.stream_of(y)))
+        assert torch.equal(y, want)
