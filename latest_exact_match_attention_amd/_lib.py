@@ -127,10 +127,16 @@ def check(status: int) -> None:
     raise RuntimeError(f"HIP error in liblema_hip: {msg}")
 
 
+# torch's own accessor of a device's current raw stream; a private name, so it may be missing
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
     """The raw hipStream_t of the current torch stream on t's device (0.1 us; a Stream object
     of current_stream() takes 1.8)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    if _RAW_STREAM is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _RAW_STREAM(t.get_device())
 
 
 # ---- host memory the GPU works on in place (a store table in host RAM) ----

@@ -234,6 +234,18 @@ def _hard_z(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 GRAD_KERNEL_T = 1 << 20
 
 
+def _unwatched(gy: torch.Tensor) -> bool:
+    """Whether no forward mode, dispatch mode or functional transform looks at operations on gy.
+    torch has no public name for these; one that is missing or renamed counts as a yes to them."""
+    try:
+        ft = torch._C._functorch
+        return (torch._C._len_torch_dispatch_stack() == 0
+                and not ft.is_functorch_wrapped_tensor(gy) and not ft.is_legacy_batchedtensor(gy)
+                and torch.autograd.forward_ad._current_level < 0 and not gy._is_zerotensor())
+    except AttributeError:
+        return False
+
+
 def _plain_grad(gy: torch.Tensor, src: torch.Tensor) -> bool:
     """Whether a backward may hand gy and the saved indices to the kernel: an ordinary device
     tensor whose own gradient nobody asks for, and the indices as they were saved (a saved-tensor
@@ -241,14 +253,10 @@ def _plain_grad(gy: torch.Tensor, src: torch.Tensor) -> bool:
     gradients and traced or otherwise wrapped tensors keep the tensor operations, which
     compose with them or refuse them by themselves. So do deterministic algorithms: the kernel
     adds a source row's gradients in the order its wavefronts list them."""
-    ft = torch._C._functorch
     return (type(gy) is torch.Tensor and type(src) is torch.Tensor and src.dtype is torch.int32
-            and src.device == gy.device and src.shape == gy.shape[:3] and gy.is_cuda and gy.dtype in _lib.DTYPE_CODE
-            and not torch.is_grad_enabled() and torch._C._len_torch_dispatch_stack() == 0
-            and not ft.is_functorch_wrapped_tensor(gy) and not ft.is_legacy_batchedtensor(gy)
-            and torch.autograd.forward_ad._current_level < 0
-            and not gy.is_neg() and not gy._is_zerotensor()
-            and not torch.are_deterministic_algorithms_enabled()
+            and src.device == gy.device and src.shape == gy.shape[:3] and gy.is_cuda
+            and gy.dtype in _lib.DTYPE_CODE and not torch.is_grad_enabled() and _unwatched(gy)
+            and not gy.is_neg() and not torch.are_deterministic_algorithms_enabled()
             and gy.shape[2] < GRAD_KERNEL_T)
 
 

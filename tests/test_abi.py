@@ -116,3 +116,22 @@ def test_noalloc_scratch_size_agrees_with_header():
     text = (ROOT / "include" / "lema_hip.h").read_text()
     m = re.search(r"#define LEMA_NOALLOC_SCRATCH_BYTES \((\d+)LL \* 1024 \* 1024\)", text)
     assert m and int(m.group(1)) * 1024 * 1024 == _lib.NOALLOC_SCRATCH_BYTES
+
+
+def test_torch_private_names_may_be_missing(monkeypatch):
+    """The names torch does not document are read with a way out: the stream of the public
+    accessor, and tensor operations for a backward nobody can vouch for."""
+    import torch
+    from types import SimpleNamespace
+
+    from latest_exact_match_attention_amd import _lib, attention
+    x = torch.zeros(3)
+    monkeypatch.setattr(_lib, "_RAW_STREAM", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: SimpleNamespace(cuda_stream=(dev, 7)))
+    assert _lib.stream_of(x) == (x.device, 7)
+    assert attention._unwatched(x)
+    for owner, name in ((torch._C, "_len_torch_dispatch_stack"), (torch._C._functorch, "is_legacy_batchedtensor"),
+                        (torch.autograd.forward_ad, "_current_level")):
+        with monkeypatch.context() as m:
+            m.delattr(owner, name)
+            assert not attention._unwatched(x)
