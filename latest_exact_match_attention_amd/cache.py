@@ -134,6 +134,7 @@ class HashStore:
                 and values.shape[3] * es == self.vbytes
                 and (values.stride(3) == 1 or values.shape[3] == 1) and values.data_ptr() % 8 == 0
                 and all(s * es % 8 == 0 for s in values.stride()[:3])
+                and not values.is_neg() and not values.is_conj()   # signs a copy would carry out
                 and (out is None or out.untyped_storage().data_ptr()
                      != values.untyped_storage().data_ptr()))
         if not view:

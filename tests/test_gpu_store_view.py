@@ -75,3 +75,19 @@ def test_results_over_the_values_memory(dev):
     b.exchange(kc, kc, base.transpose(1, 2), out, T, 0)
     assert torch.equal(out, want)
     assert _entries(a) == _entries(b)
+
+
+def test_a_view_that_carries_a_sign(dev):
+    """A negated or conjugated view's signs are not in memory: such values are copied first."""
+    g = torch.Generator().manual_seed(4)
+    B, H, T, d = 1, 2, 40, 8
+    kc = torch.randint(0, 9, (B, H, T), generator=g).to(dev)
+    z = torch.randn((B, T, H, d), generator=g, dtype=torch.complex64).to(dev)
+    for x in (torch._neg_view(z.real.contiguous()).transpose(1, 2), z.conj().transpose(1, 2)):
+        a, b = (HashStore(d * x.element_size() // 4, groups=B * H, dtype=torch.float32, capacity=4096, device=dev)
+                for _ in range(2))
+        want, got = (torch.empty((B, H, T, d), dtype=x.dtype, device=dev) for _ in range(2))
+        a.exchange(kc, kc, x.resolve_neg().resolve_conj().contiguous(), want, T, 0)
+        b.exchange(kc, kc, x, got, T, 0)
+        assert torch.equal(got, want)
+        assert _entries(a) == _entries(b)
