@@ -38,6 +38,14 @@ def _codes(t: torch.Tensor) -> tuple[torch.Tensor, int]:
     return t.contiguous(), t.element_size()
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the spans of memory from the first to the last element meet."""
+    lo = [t.data_ptr() for t in (a, b)]
+    hi = [p + t.element_size() * (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride())))
+          for p, t in zip(lo, (a, b))]
+    return lo[0] < hi[1] and lo[1] < hi[0]
+
+
 class HashStore:
     """ONE open-addressing table (linear probing, fixed capacity) for every (layer, stream,
     head) partition; an entry's key is (group, code) (code/lema/cache.py:129-201).
@@ -135,8 +143,7 @@ class HashStore:
                 and (values.stride(3) == 1 or values.shape[3] == 1) and values.data_ptr() % 8 == 0
                 and all(s * es % 8 == 0 for s in values.stride()[:3])
                 and not values.is_neg() and not values.is_conj()   # signs a copy would carry out
-                and (out is None or out.untyped_storage().data_ptr()
-                     != values.untyped_storage().data_ptr()))
+                and (out is None or not _overlap(values, out)))
         if not view:
             values = values.contiguous()
         if values.numel() * values.element_size() != n * self.vbytes:

@@ -91,3 +91,21 @@ def test_a_view_that_carries_a_sign(dev):
         b.exchange(kc, kc, x, got, T, 0)
         assert torch.equal(got, want)
         assert _entries(a) == _entries(b)
+
+
+def test_results_over_part_of_the_values_memory(dev):
+    """Overlap is a matter of addresses: tensors that share memory may have storages of their own."""
+    g = torch.Generator().manual_seed(5)
+    B, H, T, d = 2, 4, 700, 8
+    n = B * H * T * d
+    kc = torch.randint(0, 9, (B, H, T), generator=g).to(dev)
+    buf = torch.randn(n + 64, generator=g).to(dev)
+    values = buf[:n].view(B, T, H, d).transpose(1, 2)
+    out = torch.from_dlpack(buf[64:].view(B, H, T, d))
+    assert out.untyped_storage().data_ptr() != values.untyped_storage().data_ptr()
+    a, b = (HashStore(d, groups=B * H, dtype=torch.float32, capacity=1 << 14, device=dev) for _ in range(2))
+    want = torch.empty((B, H, T, d), device=dev)
+    a.exchange(kc, kc, values.contiguous(), want, T, 0)
+    b.exchange(kc, kc, values, out, T, 0)
+    assert torch.equal(out, want)
+    assert _entries(a) == _entries(b)
