@@ -16,7 +16,7 @@
 // Every row of gv is written once, zeros included. A list that fills up before the scan ends is
 // reduced at once and the rows then accumulate in gv (rounded once per list, in 16-bit types).
 // The scan reads O(T^2 / R) indices from L2, 4 bytes each: at T = 100,000 and R = 1024 about
-// 49 per index against the 48 to 256 bytes of its gy row. It counts 8192 indices behind one
+// 49 per index against the 48 to 256 bytes of its gy row. It counts 6144 indices behind one
 // barrier before it lists them: with two barriers for every batch or two of 1024, one row of
 // 131,072 positions (d_v 24 bf16) took 104 us where 39 are now.
 //
@@ -42,7 +42,7 @@ constexpr int kGgBatch = 4 * kGgThreads; // indices of a 16-byte load by every t
 constexpr int kGgList = 2560;
 constexpr int kGgFlight = 8;             // gy rows in flight per group of lanes
 constexpr int kGgSliceT = 16384;         // shorter rows' lists are short whoever reads what
-constexpr int kGgSpan = 8;               // batches of indices whose loads are issued together
+constexpr int kGgSpan = 6;               // batches of indices whose loads are issued together
 constexpr int kMissPositions = 256;      // positions per workgroup of the miss kernel
 
 struct GradArgs {
@@ -184,8 +184,10 @@ struct GradLds {
 // dead once it is sorted.
 static_assert(sizeof(int32_t) * kGgList >= sizeof(float) * 8 * kGgThreads, "the runs' first sums");
 
+// 16-byte pieces take 155 registers, 3 workgroups per CU: held to 128 a few were spilled, and the
+// scratch made every launch wait.
 template <int DTYPE, int VEC>
-__global__ __launch_bounds__(kGgThreads, 4) void gather_grad_kernel(GradArgs a) {
+__global__ __launch_bounds__(kGgThreads, VEC == 16 ? 3 : 4) void gather_grad_kernel(GradArgs a) {
   typedef GgPiece<DTYPE, VEC> P;
   constexpr int E = P::kElems;
   __shared__ GradLds s;
