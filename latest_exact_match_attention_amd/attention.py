@@ -249,15 +249,15 @@ def _unwatched(gy: torch.Tensor) -> bool:
 def _plain_grad(gy: torch.Tensor, src: torch.Tensor) -> bool:
     """Whether a backward may hand gy and the saved indices to the kernel: an ordinary device
     tensor whose own gradient nobody asks for, and the indices as they were saved (a saved-tensor
-    hook may bring them back in another type or on another device). A graph of the backward (create_graph), forward mode, batched
-    gradients and traced or otherwise wrapped tensors keep the tensor operations, which
-    compose with them or refuse them by themselves. So do deterministic algorithms: the kernel
-    adds a source row's gradients in the order its wavefronts list them."""
-    return (type(gy) is torch.Tensor and type(src) is torch.Tensor and src.dtype is torch.int32
-            and src.device == gy.device and src.shape == gy.shape[:3] and gy.is_cuda
-            and gy.dtype in _lib.DTYPE_CODE and not torch.is_grad_enabled() and _unwatched(gy)
-            and not gy.is_neg() and not torch.are_deterministic_algorithms_enabled()
-            and gy.shape[2] < GRAD_KERNEL_T)
+    hook may bring them back in another type or on another device). A graph of the backward
+    (create_graph), forward mode, batched gradients and traced or otherwise wrapped tensors keep
+    the tensor operations, which compose with them or refuse them by themselves. So do
+    deterministic algorithms: the kernel adds a source row's gradients in the order its wavefronts
+    list them."""
+    return (type(gy) is torch.Tensor and type(src) is torch.Tensor and gy.is_cuda
+            and src.dtype is torch.int32 and src.get_device() == gy.get_device()
+            and gy.dtype in _lib.DTYPE_CODE and not torch.is_grad_enabled() and not gy.is_neg()
+            and not torch.are_deterministic_algorithms_enabled() and _unwatched(gy))
 
 
 class _LemaGather(torch.autograd.Function):
@@ -277,13 +277,13 @@ class _LemaGather(torch.autograd.Function):
     def backward(ctx, gy):
         (src,) = ctx.saved_tensors
         B, H, T, dv = ctx.v_shape
-        if _plain_grad(gy, src):
-            gy = gy if gy.stride(-1) == 1 or dv == 1 else gy.contiguous()
-            gv = torch.empty((B, H, T, dv), dtype=gy.dtype, device=gy.device)
+        if T < GRAD_KERNEL_T and src.numel() == B * H * T and _plain_grad(gy, src):
+            gy = gy if gy.stride(3) == 1 or dv == 1 else gy.contiguous()
+            gv = gy.new_empty((B, H, T, dv))
+            sb, sh, st, _ = gy.stride()
             _lib.check(_lib.lib().lema_gather_grad(
-                gy.data_ptr(), _lib.DTYPE_CODE[gy.dtype], B, H, T, dv, gy.stride(0),
-                gy.stride(1), gy.stride(2), src.contiguous().data_ptr(), gv.data_ptr(),
-                _lib.stream_of(gy)))
+                gy.data_ptr(), _lib.DTYPE_CODE[gy.dtype], B, H, T, dv, sb, sh, st,
+                src.contiguous().data_ptr(), gv.data_ptr(), _lib.stream_of(gy)))
             return None, None, gv
         hit = (src >= 0).unsqueeze(-1)
         idx = src.clamp_min(0).to(torch.int64).view(B * H, T, 1).expand(B * H, T, dv)

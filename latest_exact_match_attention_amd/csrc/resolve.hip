@@ -343,8 +343,9 @@ __global__ __launch_bounds__(kThreads) void mask_kernel(ResolveArgs a) {
   if (part == 0 && threadIdx.x == 0) a.mask_built[row] = built;
   if (!built) return;
   for (int item = threadIdx.x >> 6; item < a.mask_words * kTurnRuns; item += kThreads / 64) {
-    const int cb = item / kTurnRuns;
-    const int w0 = (part * kTurnRuns + item % kTurnRuns) * kTurnWords;
+    // a run's 64-chunk blocks side by side: they write the same lines
+    const int cb = item % a.mask_words;
+    const int w0 = (part * kTurnRuns + item / a.mask_words) * kTurnWords;
     const int64_t chunk = 64 * cb + lane;
     const int ln = chunk < full ? lone[chunk] : 0;
     const bool have = ln > kLoneChunk && (ln <= kLoneQueue || a.nchunks > kMaskQueueChunks);  // as summary_kernel
