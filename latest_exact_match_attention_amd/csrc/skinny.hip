@@ -135,8 +135,9 @@ __device__ __forceinline__ u32x4 swap_halves(u32x4 v) {
 // them. U is the K-steps of a group (kHalf: pairs of steps). A wavefront whose share is more than
 // a group (kMore) issues the next group's loads before the current one's products, so it has
 // one to two groups in flight. With a pre-norm one group is all of its share (3, 4, 6 or 8 steps
-// for K of up to 768, 1024, 1536 or 2048), and the weights' loads are issued before the
-// pre-norm's arithmetic and arrive meanwhile. Steps past the share cost a load each, and a second
+// for K of up to 768, 1024, 1536 or 2048; gate and up beyond 1536 take two of 4, whose registers
+// leave room for a second workgroup: K 1792, 16 rows 22.0 -> 18.6 us), and the weights' loads are
+// issued before the pre-norm's arithmetic and arrive meanwhile. Steps past the share cost a load each, and a second
 // group's registers keep other workgroups off the CU: K = 768, N = 50304 (3 steps) took
 // 22.6 us at M = 1 and 42.6 at M = 17 with groups of 4 and room for two, 14.8 and 24.4 now
 // (16.4 and 27.4 with every load conditional).
@@ -155,8 +156,7 @@ __device__ __forceinline__ u32x4 swap_halves(u32x4 v) {
 // 3.64 and 5.14.)
 template <int MT, int CT, int kNorm, int U, bool kHalf, bool kMore>
 __global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 4 : 2) void skinny_kernel(SkDevice a) {
-  constexpr int kSteps = (kSkStepK * U + 511) / 512;  // the norm's, of 512 elements
-  static_assert(kNorm == 0 || !kMore, "one group of loads");
+  constexpr int kSteps = (kSkStepK * U * (kMore ? 2 : 1) + 511) / 512;  // the norm's, of 512 elements
   static_assert(!kHalf || (MT == 1 && CT == 1 && kNorm == 0), "a half-filled tile");
   __shared__ float part[kSkWaves][MT * 16][CT * 16 + 1];
   extern __shared__ __align__(16) uint16_t xs[];  // kNorm: the normalised rows, stride K + 8
@@ -491,7 +491,11 @@ int launch_skinny(SkinnyArgs& a, hipStream_t st) {
         if (per <= 3) return skinny_kernel<MT, CT, kNorm, 3, false, false>;
         if (per <= 4) return skinny_kernel<MT, CT, kNorm, 4, false, false>;
       }
-      return per <= 6 ? skinny_kernel<MT, CT, kNorm, 6, false, false> : skinny_kernel<MT, CT, kNorm, 8, false, false>;
+      if (per <= 6) return skinny_kernel<MT, CT, kNorm, 6, false, false>;
+      if constexpr (CT == 2)
+        return skinny_kernel<MT, CT, kNorm, 4, false, true>;
+      else
+        return skinny_kernel<MT, CT, kNorm, 8, false, false>;
     };
     auto pick = [&](auto mt) {
       return a.nd != nullptr ? pick_u(mt, std::integral_constant<int, 2>{}) : pick_u(mt, std::integral_constant<int, 1>{});
