@@ -79,9 +79,9 @@ struct SkinnyArgs {
   float eps;
 };
 
-// What the kernel gets of it: two cache lines of arguments, the first one all that a plain
+// What the kernel gets of it: two lines of 64 bytes of arguments, the first one all that a plain
 // product needs. The argument lines are cold at every launch, and the weights' loads wait for
-// them (with the four lines of SkinnyArgs every launch took 0.3 to 0.5 us more).
+// them (in five lines of 64 bytes, as they were before, every launch took 0.3 to 0.5 us more).
 struct SkDevice {
   const uint16_t* x;
   const uint16_t* w;
@@ -102,7 +102,7 @@ struct SkDevice {
   float eps;
   int32_t d, T, Nv;
 };
-static_assert(sizeof(SkDevice) == 128, "two cache lines");
+static_assert(sizeof(SkDevice) == 128, "two lines");
 
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
   const uint32_t b = __float_as_uint(f);
@@ -155,7 +155,7 @@ __device__ __forceinline__ u32x4 swap_halves(u32x4 v) {
 // 6.96 and 5.16; M = 16, N = 8192 10.9 and 8.9. (Half-filled tiles whose steps were summed apart:
 // 3.64 and 5.14.)
 template <int MT, int CT, int kNorm, int U, bool kHalf, bool kMore>
-__global__ __launch_bounds__(kSkThreads, kNorm != 0 && U <= 6 && MT * CT <= 2 ? 4 : 2) void skinny_kernel(SkDevice a) {
+__global__ __launch_bounds__(kSkThreads, MT * CT <= 2 && (kNorm != 0 ? U <= 6 : !kMore || U <= 4) ? 4 : 2) void skinny_kernel(SkDevice a) {
   constexpr int kSteps = (kSkStepK * U * (kMore ? 2 : 1) + 511) / 512;  // the norm's, of 512 elements
   static_assert(!kHalf || (MT == 1 && CT == 1 && kNorm == 0), "a half-filled tile");
   __shared__ float part[kSkWaves][MT * 16][CT * 16 + 1];
@@ -501,34 +501,33 @@ int launch_skinny(SkinnyArgs& a, hipStream_t st) {
       return a.nd != nullptr ? pick_u(mt, std::integral_constant<int, 2>{}) : pick_u(mt, std::integral_constant<int, 1>{});
     };
     kernel = a.M <= 16 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
-  } else if constexpr (CT == 1) {
-    // steps past a share of `n` in groups of u; the larger group unless it divides the share worse
-    auto waste = [](int n, int u) { return (n + u - 1) / u * u - n; };
-    const int half = (per + 1) / 2;  // pairs of steps
-    auto pick = [&](auto mt) {
-      constexpr int MT = decltype(mt)::value;
-      if (per <= 3) return skinny_kernel<MT, 1, 0, 3, false, false>;
-      if (per <= 4) return skinny_kernel<MT, 1, 0, 4, false, false>;
-      if (per <= 6) return skinny_kernel<MT, 1, 0, 6, false, false>;
-      return waste(per, 6) <= waste(per, 4) ? skinny_kernel<MT, 1, 0, 6, false, true> : skinny_kernel<MT, 1, 0, 4, false, true>;
-    };
-    if (narrow && a.M <= 8 && a.K >= 64)
-      kernel = half <= 2   ? skinny_kernel<1, 1, 0, 2, true, false>
-               : half <= 3 ? skinny_kernel<1, 1, 0, 3, true, false>
-               : half <= 4 ? skinny_kernel<1, 1, 0, 4, true, false>
-               : waste(half, 4) <= waste(half, 3) ? skinny_kernel<1, 1, 0, 4, true, true> : skinny_kernel<1, 1, 0, 3, true, true>;
-    else
-      kernel = a.M <= 16 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
   } else {
+    // A share of up to 6 steps in one group; longer ones in groups of 4, or of 6 where that divides
+    // the share as well and two groups' registers still leave room for a second workgroup.
+    auto waste = [](int n, int u) { return (n + u - 1) / u * u - n; };  // loads past a share of n
     auto pick = [&](auto mt) {
       constexpr int MT = decltype(mt)::value;
-      if constexpr (CT == 2) {
-        if (per <= 3) return skinny_kernel<MT, CT, 0, 3, false, false>;
-        if (per <= 4) return skinny_kernel<MT, CT, 0, 4, false, false>;
+      if constexpr (CT <= 2) {
+        if (per <= 2) return skinny_kernel<MT, CT, 0, 2, false, false>;
+      }
+      if (per <= 3) return skinny_kernel<MT, CT, 0, 3, false, false>;
+      if (per <= 4) return skinny_kernel<MT, CT, 0, 4, false, false>;
+      if (per <= 6) return skinny_kernel<MT, CT, 0, 6, false, false>;
+      if constexpr (MT * CT == 1) {
+        if (waste(per, 6) <= waste(per, 4)) return skinny_kernel<MT, CT, 0, 6, false, true>;
       }
       return skinny_kernel<MT, CT, 0, 4, false, true>;
     };
     kernel = a.M <= 16 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
+    if constexpr (CT == 1) {
+      const int half = (per + 1) / 2;  // pairs of steps
+      if (narrow && a.M <= 8 && a.K >= 64)
+        kernel = half <= 2   ? skinny_kernel<1, 1, 0, 2, true, false>
+                 : half <= 3 ? skinny_kernel<1, 1, 0, 3, true, false>
+                 : half <= 4 ? skinny_kernel<1, 1, 0, 4, true, false>
+                 : waste(half, 4) <= waste(half, 3) ? skinny_kernel<1, 1, 0, 4, true, true>
+                                                    : skinny_kernel<1, 1, 0, 3, true, true>;
+    }
   }
   kernel<<<grid, block, lds, st>>>(g);
   return launch_status("skinny_kernel");
@@ -538,8 +537,7 @@ int launch_ct(SkinnyArgs& a, int ct, hipStream_t st) {
   switch (ct) {
     case 1: return launch_skinny<1>(a, st);
     case 2: return launch_skinny<2>(a, st);
-    case 3: return launch_skinny<3>(a, st);
-    default: return launch_skinny<4>(a, st);
+    default: return launch_skinny<3>(a, st);
   }
 }
 
@@ -561,11 +559,11 @@ int check_weight(const void* w, int64_t N) {
 
 // Column tiles per block for codes of d bits: one (16 columns, a head split over blocks
 // writes its bytes from each) when d is a multiple of 8, else the least multiple of 16 (up to
-// 64) holding whole heads, or 0. More blocks of fewer weight rows: the q and k projections of
+// 48) holding whole heads, or 0. More blocks of fewer weight rows: the q and k projections of
 // 64-bit heads ran on 24 blocks of 64 rows each.
 int pack_ct(int32_t d) {
   if (d % 8 == 0) return 1;
-  for (int c = 1; c <= 4; ++c)
+  for (int c = 1; c <= 3; ++c)
     if ((16 * c) % d == 0) return c;
   return 0;
 }
