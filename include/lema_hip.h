@@ -75,9 +75,11 @@ int lema_hard(const void* qc, const void* kc, int32_t code_bytes, const void* v,
               int32_t miss, void* src, int32_t src_bytes, void* stream);
 
 /* Workspace bytes lema_latest_prev_match_ws and lema_hard_ws use for N rows of T positions:
- * about 24 KB per 1024 positions, 0 for rows of fewer than 64,513 positions (64 chunks of 1024;
- * shorter rows keep the backward scan, which is faster there, and need none). No reference counterpart: the reference's sort needs no scratch the
- * caller provides. */
+ * per row 16 KB for each started chunk of 1024 (its summary and its code bits), 512 KB for each
+ * started 64 chunks (the bits turned round) and a few bytes a chunk, so 24 to 32 KB per 1024
+ * positions; 0 for rows of fewer than 64,513 positions (64 chunks; shorter rows keep the backward
+ * scan, which is faster there, and need none). No reference counterpart: the reference's sort
+ * needs no scratch the caller provides. */
 int64_t lema_resolve_workspace_bytes(int64_t N, int64_t T);
 
 /* lema_latest_prev_match and lema_hard with a workspace (256-byte aligned, at least
@@ -117,8 +119,9 @@ int lema_gather(const void* v, int32_t dtype, int64_t B, int64_t H, int64_t T, i
                 void* stream);
 
 /* The gradient of the gather: gv[b, h, j, :] = sum of gy[b, h, i, :] over the queries i with
- * src[b, h, i] = j, summed in fp32 and rounded once (16-bit types: once per 1536 or more listed
- * queries of 1024 rows). A missed query's row times zero counts towards row 0, so an infinity
+ * src[b, h, i] = j, summed in fp32 in no fixed order and rounded once (16-bit types: once per 1536
+ * or more listed queries of 1024 rows). Its time grows with the square of T: every index is read
+ * once for each 1024 source rows. A missed query's row times zero counts towards row 0, so an infinity
  * or NaN there makes that column of gv[b, h, 0] NaN. Replaces the backward of
  * code/lema/attention.py:157-158.
  *   gy   [B, H, T, dv] of `dtype`, element strides (any, zero included), last dim contiguous

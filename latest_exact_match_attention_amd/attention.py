@@ -101,7 +101,7 @@ def latest_prev_match(qc: torch.Tensor, kc: torch.Tensor,
 
 def resolve_workspace(N: int, T: int, device) -> torch.Tensor | None:
     """Scratch for the chunk summaries of N rows of T positions (None when rows are short
-    enough for the backward scan): about 24 KB per 1024 positions."""
+    enough for the backward scan): 24 to 32 KB per 1024 positions."""
     n = _lib.lib().lema_resolve_workspace_bytes(N, T)
     return torch.empty(n, dtype=torch.uint8, device=device) if n > 0 else None
 
