@@ -38,14 +38,6 @@ def _codes(t: torch.Tensor) -> tuple[torch.Tensor, int]:
     return t.contiguous(), t.element_size()
 
 
-def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
-    """Whether the spans of memory from the first to the last element meet."""
-    lo = [t.data_ptr() for t in (a, b)]
-    hi = [p + t.element_size() * (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride())))
-          for p, t in zip(lo, (a, b))]
-    return lo[0] < hi[1] and lo[1] < hi[0]
-
-
 class HashStore:
     """ONE open-addressing table (linear probing, fixed capacity) for every (layer, stream,
     head) partition; an entry's key is (group, code) (code/lema/cache.py:129-201).
@@ -134,16 +126,20 @@ class HashStore:
         if g0 < 0 or g0 + n // T > self.groups:
             raise ValueError(f"groups [{g0}, {g0 + n // T}) outside the store's {self.groups}")
         _lib.require_device(kc, values)
-        # a [B, H, T, d] view (a projection's values) is read in place where its strides allow and
-        # the results go to other memory
-        es = values.element_size()
-        view = (T > 1 and values.dim() == 4 and not values.is_contiguous() and values.shape[2] == T
-                and n > 0 and values.shape[0] * values.shape[1] * T == n
-                and values.shape[3] * es == self.vbytes
-                and (values.stride(3) == 1 or values.shape[3] == 1) and values.data_ptr() % 8 == 0
-                and all(s * es % 8 == 0 for s in values.stride()[:3])
-                and not values.is_neg() and not values.is_conj()   # signs a copy would carry out
-                and (out is None or not _overlap(values, out)))
+        # a [B, H, T, d] view (a projection's values) is read in place where its strides allow, its
+        # values are what lies in memory (no negated or conjugated view) and the results go to other
+        # memory
+        view = T > 1 and n > 0 and values.dim() == 4 and not values.is_contiguous()
+        if view:
+            (B, H, Tv, d), (sb, sh, st, sd) = values.shape, values.stride()
+            es, at = values.element_size(), values.data_ptr()
+            view = (Tv == T and B * H * T == n and d * es == self.vbytes and (sd == 1 or d == 1)
+                    and (at | (sb | sh | st) * es) % 8 == 0
+                    and not values.is_neg() and not values.is_conj())
+            if view and out is not None:
+                end = at + es * (1 + (B - 1) * sb + (H - 1) * sh + (T - 1) * st + (d - 1) * sd)
+                to = out.data_ptr()
+                view = to >= end or to + out.numel() * out.element_size() <= at
         if not view:
             values = values.contiguous()
         if values.numel() * values.element_size() != n * self.vbytes:
@@ -163,11 +159,9 @@ class HashStore:
         tail = (self.counts_device.data_ptr(), self.full_flag.data_ptr(),
                 ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_of(kc))
         if view:
-            B, H = values.shape[:2]
-            sb, sh, st = (s * es for s in values.stride()[:3])
             _lib.check(L.lema_store_exchange_view(
-                table, self.cap, self.vbytes, qp, kc.data_ptr(), cb, values.data_ptr(), B, H, sb,
-                sh, st, outp, T, g0, *tail))
+                table, self.cap, self.vbytes, qp, kc.data_ptr(), cb, at, B, H, sb * es, sh * es,
+                st * es, outp, T, g0, *tail))
         else:
             _lib.check(L.lema_store_exchange_ws(
                 table, self.cap, self.vbytes, qp, kc.data_ptr(), cb, values.data_ptr(), outp, n, T,
